@@ -399,6 +399,22 @@ int starkv_prefill_attention(void *stream, const void *query, int64_t q_s0, int6
                              int out_dtype);
 
 /*
+ * The lift in front of the dense prefill (the reference's batched product and RoPE,
+ * starkv_serve/attention.py:219-241): from the step's codes (k_codes [T, k_width] and v_codes
+ * [T, v_rank], element row strides, one dtype: bf16, fp16 or fp32), key [T, num_kv_heads, 128]
+ * fp16 = RoPE(codes @ U) at each token's position in its prompt, formed in fp32 and rounded
+ * once, and, with v_out, the bf16 or fp32 V codes in fp16, rows of v_rank elements. k_up: U in
+ * fp32, rank-major (element row stride u_s0); the heads' widths and offsets int32 on the device.
+ * cos_sin [positions, 128] = cos | sin (bf16, fp16 or fp32, row stride cs_s0) must cover the
+ * longest prompt.
+ */
+int starkv_prefill_lift(void *stream, const void *k_codes, int64_t k_s0, const void *v_codes, int64_t v_s0,
+                        int code_dtype, int num_tokens, const int32_t *cu_seqlens, int num_prompts,
+                        const float *k_up, int64_t u_s0, const int32_t *k_offsets, const int32_t *k_widths,
+                        int num_kv_heads, const void *cos_sin, int64_t cs_s0, int cs_dtype, void *key, void *v_out,
+                        int v_rank);
+
+/*
  * Timing for benchmarks (no counterpart in the reference, whose benchmark reads profiler
  * traces instead, bench_serving.py:71-115). starkv_profile_begin arms up to max_calls
  * event pairs; each following decode call records one pair on its stream, around its

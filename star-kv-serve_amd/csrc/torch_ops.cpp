@@ -237,6 +237,33 @@ void prefill(const at::Tensor& query, const at::Tensor& key, const at::Tensor& v
           "prefill");
 }
 
+// K lifted and rotated from the step's codes, V codes to fp16 rows (attention.py:219-241).
+void prefill_lift(const at::Tensor& k_codes, const at::Tensor& v_codes, const at::Tensor& cu_seqlens,
+                  const at::Tensor& k_up, const at::Tensor& k_offsets, const at::Tensor& k_widths,
+                  const at::Tensor& cos_sin, const at::Tensor& key, const std::optional<at::Tensor>& v_out) {
+    const c10::DeviceGuard guard(k_codes.device());
+    TORCH_CHECK(k_up.scalar_type() == at::kFloat && k_up.size(1) == 128 && k_up.stride(1) == 1,
+                "starkv.prefill_lift: k_up must be fp32 rows of 128");
+    TORCH_CHECK(k_codes.size(1) == k_up.size(0) && k_offsets.numel() == k_widths.numel() && k_codes.stride(1) == 1 &&
+                    v_codes.stride(1) == 1 && v_codes.size(0) == k_codes.size(0) && cos_sin.size(1) == 128 &&
+                    cos_sin.stride(1) == 1,
+                "starkv.prefill_lift: shapes");
+    TORCH_CHECK(!v_out || v_codes.scalar_type() == k_codes.scalar_type(), "starkv.prefill_lift: codes must share one dtype");
+    TORCH_CHECK(key.is_contiguous() && key.scalar_type() == at::kHalf && key.size(0) == k_codes.size(0) &&
+                    key.size(1) == k_offsets.numel() && key.size(2) == 128,
+                "starkv.prefill_lift: key must be contiguous fp16 [T, heads, 128]");
+    TORCH_CHECK(!v_out || (v_out->is_contiguous() && v_out->scalar_type() == at::kHalf &&
+                           v_out->sizes() == v_codes.sizes()),
+                "starkv.prefill_lift: v_out must be contiguous fp16 [T, v_rank]");
+    check(starkv_prefill_lift(stream_of(k_codes), k_codes.data_ptr(), k_codes.stride(0), v_codes.data_ptr(),
+                              v_codes.stride(0), dtype_code(k_codes), (int)k_codes.size(0),
+                              i32(cu_seqlens, "cu_seqlens"), (int)cu_seqlens.numel() - 1, k_up.data_ptr<float>(),
+                              k_up.stride(0), i32(k_offsets, "k_offsets"), i32(k_widths, "k_widths"),
+                              (int)k_offsets.numel(), cos_sin.data_ptr(), cos_sin.stride(0), dtype_code(cos_sin),
+                              key.data_ptr(), v_out ? v_out->data_ptr() : nullptr, (int)v_codes.size(1)),
+          "prefill_lift");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(starkv, m) {
@@ -260,6 +287,8 @@ TORCH_LIBRARY(starkv, m) {
     m.def("stock_write(Tensor key, Tensor value, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping) -> ()");
     m.def("prefill(Tensor query, Tensor key, Tensor value, Tensor cu_seqlens, Tensor blocks, float scale, "
           "Tensor(a!) out) -> ()");
+    m.def("prefill_lift(Tensor k_codes, Tensor v_codes, Tensor cu_seqlens, Tensor k_up, Tensor k_offsets, "
+          "Tensor k_widths, Tensor cos_sin, Tensor(a!) key, Tensor(b!)? v_out) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(starkv, CUDA, m) {
@@ -272,4 +301,5 @@ TORCH_LIBRARY_IMPL(starkv, CUDA, m) {
     m.impl("stock_decode", &stock_decode);
     m.impl("stock_write", &stock_write);
     m.impl("prefill", &prefill);
+    m.impl("prefill_lift", &prefill_lift);
 }

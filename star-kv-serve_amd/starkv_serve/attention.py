@@ -48,7 +48,7 @@ from starkv_serve.checkpoint import StarKVLayerWeights, layer_operands
 from starkv_serve.kernels.kv_write import flush_write, write_codes, write_kv
 from starkv_serve.kernels.paged_decode import paged_starkv_decode
 from starkv_serve.kernels.paged_quant import HEAD_DIM, pack_kv, paged_quant_decode
-from starkv_serve.kernels.prefill import prefill_attention
+from starkv_serve.kernels.prefill import prefill_attention, prefill_lift, prompt_tables
 
 DECODER = "decoder"  # AttentionType.DECODER
 
@@ -185,23 +185,13 @@ class StarKVAttentionImpl:
         self.kv_groups = ops.kv_groups
         if self.row is not None:
             self.k_nouts, self.head_of_lane, self.k_tiles = ops.k_nouts, ops.head_of_lane, ops.k_tiles
-        # Prefill lifts every KV head in one batched product, which needs one width: the
-        # codes are gathered into a padded [T, H, R] view. Lanes past a head's width point
-        # at its first code; the rows of U they meet are zero (attention.py:144-160).
-        w, H, Hd = self.w, self.num_kv_heads, self.head_size
-        R = w.k_max_rank
-        idx = torch.empty(H * R, dtype=torch.long)
-        k_up_pad = torch.zeros(H, R, Hd, dtype=w.k_up.dtype)
-        for h, (off, width) in enumerate(zip(w.k_head_offsets.tolist(), w.k_head_widths.tolist())):
-            idx[h * R:h * R + width] = torch.arange(off, off + width)
-            idx[h * R + width:(h + 1) * R] = off
-            k_up_pad[h, :width] = w.k_up[off:off + width]
-        self.k_prefill_gather = idx.to(device)
+        # The prompts' lift multiplies in fp32, heads at their own widths.
+        self.k_head_widths = self.w.k_head_widths.to(device)
+        self.k_up_f32 = self.w.k_up.to(device).float().contiguous()
         # The decode kernels read an fp16 cos/sin table: converted once here, not per step.
         self.cos_sin16 = self.rotary_emb.cos_sin_cache.to(device=device, dtype=torch.float16).contiguous()
-        self.k_up_T = k_up_pad.to(device=device, dtype=torch.float32).contiguous()
         # V's lift runs as an fp16 GEMM (fp32 accumulation, the result rounded once to fp16).
-        self.v_up_f16 = w.v_up.to(device=device, dtype=torch.float16).contiguous()  # [H * Hd, v_rank]
+        self.v_up_f16 = self.w.v_up.to(device=device, dtype=torch.float16).contiguous()  # [H * Hd, v_rank]
 
     def _cache(self, kv_cache: torch.Tensor) -> torch.Tensor:
         cache = kv_cache.squeeze(1) if kv_cache.dim() == 4 else kv_cache  # [num_blocks, block_size, width]
@@ -262,16 +252,21 @@ class StarKVAttentionImpl:
         fp16, accumulated in fp32), then causal attention of every prompt to itself on this
         library's prefill kernel. q and out [T, H_q, 128]."""
         T = q.shape[0]
-        H, R, Hd = self.num_kv_heads, self.w.k_max_rank, self.head_size
-        pos = torch.cat([torch.arange(L) for L in query_lens]).to(q.device)
-        kp = k_codes[:, self.k_prefill_gather].float().view(T, H, R).transpose(0, 1).contiguous()
-        k = torch.bmm(kp, self.k_up_T).transpose(0, 1)                                     # [T, H, Hd] fp32
-        cos, sin = self.rotary_emb.cos_sin_cache[pos].float().chunk(2, dim=-1)
-        cos, sin = cos.unsqueeze(1), sin.unsqueeze(1)
-        k1, k2 = k.chunk(2, dim=-1)
-        k = torch.cat([k1 * cos - k2 * sin, k2 * cos + k1 * sin], dim=-1).to(torch.float16)
-        v = F.linear(v_codes.to(torch.float16), self.v_up_f16).view(T, H, Hd)
-        prefill_attention(q, k, v, query_lens, self.scale, out=out)
+        if sum(query_lens) != T:
+            raise ValueError(f"prompts of {sum(query_lens)} tokens in all, {T} given")
+        if T == 0:
+            return
+        cs = self.rotary_emb.cos_sin_cache
+        if cs.dtype not in (torch.bfloat16, torch.float16, torch.float32) or cs.stride(-1) != 1:
+            cs = cs.float().contiguous()
+        if cs.shape[0] < max(query_lens) or cs.shape[1] != self.head_size:
+            raise IndexError(f"a prompt of {max(query_lens)} tokens needs more than the rotary table {tuple(cs.shape)}")
+        k_codes, v_codes = (c if c.stride(-1) == 1 else c.contiguous() for c in (k_codes, v_codes))
+        tables = prompt_tables(query_lens, q.device)
+        k, v_codes = prefill_lift(k_codes, v_codes, tables[0], self.k_up_f32, self.k_head_offsets, self.k_head_widths,
+                                  cs)
+        v = F.linear(v_codes, self.v_up_f16).view(T, self.num_kv_heads, self.head_size)
+        prefill_attention(q, k, v, query_lens, self.scale, out=out, tables=tables)
 
     def write_from_hidden(self, hidden: torch.Tensor, kv_cache: torch.Tensor, slot_mapping: torch.Tensor,
                           return_codes: bool = False, deferred: bool = False) -> Optional[torch.Tensor]:
