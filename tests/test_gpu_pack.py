@@ -118,3 +118,40 @@ def test_fold_q_matches_oracle(cuda, qdt, udt):
     assert got.shape == want.shape and ab.dtype == torch.float16
     err = np.abs(got - want)
     assert np.all(err <= np.abs(want) * 2.0 ** -10 + 1e-6), float(err.max())
+
+
+@pytest.mark.parametrize("width,off,gap", [(2160, 0, 0), (2170, 0, 0), (2159, 1, 0), (16, 0, 4), (3, 0, 0)])
+def test_write_codes_piece_sizes(cuda, width, off, gap):
+    """Rows, strides and starts that are multiples of 16, 4 and 2 bytes, more pieces than one
+    round of lanes holds and fewer: equal to index_put, nothing beside the slots touched."""
+    from starkv_serve.kernels.kv_write import write_codes
+    g = torch.Generator().manual_seed(width)
+    n, nb, W = 70, 6, width * 4 // 10
+    codes = torch.randn(n, width + off, generator=g).to(torch.bfloat16).to(cuda)[:, off:]
+    slots = torch.randperm((nb - 1) * 16, generator=g)[:n].to(cuda) + 16
+    buf = torch.randn(nb, 16, width + gap, generator=g).to(torch.bfloat16).to(cuda)
+    want = buf.clone()
+    want[slots // 16, slots % 16, :width] = codes
+    write_codes(codes[:, :W], codes[:, W:], buf[:, :, :width], slots)
+    assert torch.equal(buf.view(torch.int16), want.view(torch.int16))
+
+
+def test_pack_kv_rows_too_long_for_lds_and_lanes_no_head_holds(cuda):
+    """A V latent past one workgroup's LDS takes the form that reads codes from memory; K lanes
+    that no head holds keep the bytes the cache had."""
+    for ranks, offsets, W, R, dt in (([16, 32], [0, 16], 48, 40000, torch.bfloat16),
+                                     ([16, 20], [0, 48], 96, 33, torch.bfloat16), ([16], [16], 48, 5, torch.float32)):
+        row = pq.QuantRow(W, len(ranks), R)
+        nouts = [ref.n_outlier(r) for r in ranks]
+        g = torch.Generator().manual_seed(R)
+        k, v = torch.randn(3, W, generator=g).to(dt), torch.randn(3, R, generator=g).to(dt)
+        init = torch.randint(0, 256, (2, 16, row.nbytes), generator=g, dtype=torch.uint8)
+        slots = torch.tensor([17, 20, 31])
+        want = init.clone().numpy()
+        cquant.pack_kv(k.float().numpy(), v.float().numpy(), want, slots.numpy(), ranks, offsets, nouts, R, row.ks_off,
+                       row.vs_off, row.vq_off)
+        cache = init.to(cuda)
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=cuda)  # noqa: E731
+        pq.pack_kv(k.to(cuda), v.to(cuda), cache, slots.to(cuda), row, i32(ranks), i32(offsets), i32(nouts))
+        end = row.vq_off + row.v_bytes
+        assert np.array_equal(cache.cpu().numpy()[:, :, :end], want[:, :, :end])
