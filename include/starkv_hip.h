@@ -399,6 +399,15 @@ int starkv_prefill_attention(void *stream, const void *query, int64_t q_s0, int6
                              int out_dtype);
 
 /*
+ * Keys and values [T, num_kv_heads, 128] of bf16 or fp32 (one dtype, each its own element strides,
+ * last dimension contiguous) as the contiguous fp16 tensors starkv_prefill_attention takes, in one
+ * launch.
+ */
+int starkv_prefill_to_half(void *stream, const void *key, int64_t k_s0, int64_t k_s1, void *key_out,
+                           const void *value, int64_t v_s0, int64_t v_s1, void *value_out, int dtype, int num_tokens,
+                           int num_kv_heads);
+
+/*
  * The lift in front of the dense prefill (the reference's batched product and RoPE,
  * starkv_serve/attention.py:219-241): from the step's codes (k_codes [T, k_width] and v_codes
  * [T, v_rank], element row strides, one dtype: bf16, fp16 or fp32), key [T, num_kv_heads, 128]

@@ -237,6 +237,22 @@ void prefill(const at::Tensor& query, const at::Tensor& key, const at::Tensor& v
           "prefill");
 }
 
+// K and V [T, H, 128] of one dtype (bf16 or fp32) as contiguous fp16.
+void prefill_to_half(const at::Tensor& key, const at::Tensor& value, const at::Tensor& key_out,
+                     const at::Tensor& value_out) {
+    const c10::DeviceGuard guard(key.device());
+    TORCH_CHECK(key.scalar_type() == value.scalar_type() && key.sizes() == value.sizes() && key.dim() == 3 &&
+                    key.size(2) == 128 && key.stride(2) == 1 && value.stride(2) == 1,
+                "starkv.prefill_to_half: K and V [T, heads, 128] of one dtype");
+    for (const auto* o : {&key_out, &value_out})
+        TORCH_CHECK(o->is_contiguous() && o->scalar_type() == at::kHalf && o->sizes() == key.sizes(),
+                    "starkv.prefill_to_half: the results are contiguous fp16 of the same shape");
+    check(starkv_prefill_to_half(stream_of(key), key.data_ptr(), key.stride(0), key.stride(1), key_out.data_ptr(),
+                                 value.data_ptr(), value.stride(0), value.stride(1), value_out.data_ptr(),
+                                 dtype_code(key), (int)key.size(0), (int)key.size(1)),
+          "prefill_to_half");
+}
+
 // K lifted and rotated from the step's codes, V codes to fp16 rows (attention.py:219-241).
 void prefill_lift(const at::Tensor& k_codes, const at::Tensor& v_codes, const at::Tensor& cu_seqlens,
                   const at::Tensor& k_up, const at::Tensor& k_offsets, const at::Tensor& k_widths,
@@ -287,6 +303,7 @@ TORCH_LIBRARY(starkv, m) {
     m.def("stock_write(Tensor key, Tensor value, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping) -> ()");
     m.def("prefill(Tensor query, Tensor key, Tensor value, Tensor cu_seqlens, Tensor blocks, float scale, "
           "Tensor(a!) out) -> ()");
+    m.def("prefill_to_half(Tensor key, Tensor value, Tensor(a!) key_out, Tensor(b!) value_out) -> ()");
     m.def("prefill_lift(Tensor k_codes, Tensor v_codes, Tensor cu_seqlens, Tensor k_up, Tensor k_offsets, "
           "Tensor k_widths, Tensor cos_sin, Tensor(a!) key, Tensor(b!)? v_out) -> ()");
 }
@@ -301,5 +318,6 @@ TORCH_LIBRARY_IMPL(starkv, CUDA, m) {
     m.impl("stock_decode", &stock_decode);
     m.impl("stock_write", &stock_write);
     m.impl("prefill", &prefill);
+    m.impl("prefill_to_half", &prefill_to_half);
     m.impl("prefill_lift", &prefill_lift);
 }

@@ -55,6 +55,7 @@ SIGNATURES = {
     "starkv_prefill_block_list": (_I, [ctypes.POINTER(ctypes.c_int32), _I, ctypes.POINTER(ctypes.c_int32), _I]),
     "starkv_prefill_attention": (_I, [_P, _P, _I64, _I64, _I, _P, _P, _I64, _I64, _I, _P, _P, _I, _I, _I, _I, _F,
                                       _P, _I64, _I64, _I]),
+    "starkv_prefill_to_half": (_I, [_P, _P, _I64, _I64, _P, _P, _I64, _I64, _P, _I, _I, _I]),
     "starkv_prefill_lift": (_I, [_P, _P, _I64, _P, _I64, _I, _I, _P, _I, _P, _I64, _P, _P, _I, _P, _I64, _I, _P,
                                  _P, _I]),
     "starkv_profile_begin": (_I, [_I, _I]),

@@ -66,7 +66,8 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, query_l
 
     q [T, H_q, 128] (bf16, fp16 or fp32); k, v [T, H_kv, 128] (converted to fp16 once
     here when they are not); query_lens: the prompts' token counts (host ints, summing to
-    T); tables: their ``prompt_tables``, when the caller has them. Returns ``out`` [T, H_q, 128] (new, in q's dtype, when not given)."""
+    T); tables: their ``prompt_tables``, when the caller has them. Returns ``out``
+    [T, H_q, 128] (new, in q's dtype, when not given)."""
     T, Hq, D = q.shape
     assert D == 128 and k.shape == v.shape and k.shape[0] == T and k.shape[2] == D and Hq % k.shape[1] == 0
     assert sum(query_lens) == T
@@ -75,10 +76,11 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, query_l
     if T == 0:
         return out
     _hip.require_cuda(q, k, v, out)
-    if k.dtype != torch.float16:
-        k = k.to(torch.float16)
-    if v.dtype != torch.float16:
-        v = v.to(torch.float16)
+    if k.dtype == v.dtype and k.dtype in (torch.bfloat16, torch.float32) and k.stride(-1) == v.stride(-1) == 1:
+        kv = torch.empty((2, *k.shape), dtype=torch.float16, device=k.device)
+        _hip.ops().prefill_to_half(k, v, kv[0], kv[1])
+        k, v = kv[0], kv[1]
+    k, v = k.to(torch.float16), v.to(torch.float16)
     q = q if q.stride(-1) == 1 else q.contiguous()
     k, v = k.contiguous(), v.contiguous()
     cu_d, blk_d = prompt_tables(query_lens, q.device) if tables is None else tables

@@ -93,3 +93,28 @@ def test_prefill_bf16_kv_converted(cuda):
     out = prefill_attention(q.to(cuda), kb.to(cuda), vb.to(cuda), lengths, 0.08)
     torch.cuda.synchronize()
     assert_close(out, _truth(q, kb.half(), vb.half(), lengths, 0.08), "prefill bf16 kv")
+
+
+@pytest.mark.parametrize("kdt,vdt,how", [(torch.bfloat16, torch.bfloat16, "packed"), (torch.float32, torch.float32, "packed"),
+                                         (torch.bfloat16, torch.bfloat16, "odd"), (torch.bfloat16, torch.float16, "packed"),
+                                         (torch.bfloat16, torch.bfloat16, "dims")])
+def test_prefill_converts_keys_and_values(cuda, kdt, vdt, how):
+    """K and V of other dtypes, as slices of one projection (their own strides), at rows no wide
+    load can take ("odd") and with a strided last dimension: the same bits as fp16 copies."""
+    g = torch.Generator().manual_seed(5)
+    T, Hq, Hkv = 77, 6, 3
+    q = torch.randn(T, Hq, D, generator=g).to(torch.bfloat16).to(cuda)
+    if how == "dims":
+        kv = torch.randn(T, 2 * Hkv, 2 * D, generator=g).to(cuda)[:, :, ::2]
+    else:
+        pad = 3 if how == "odd" else 8
+        kv = torch.randn(T, 2 * Hkv * D + pad, generator=g).to(cuda)
+    k, v = kv.to(kdt), kv.to(vdt)
+    if how == "dims":
+        k, v = k[:, :Hkv], v[:, Hkv:]
+    else:
+        k = k[:, :Hkv * D].unflatten(1, (Hkv, D))
+        v = v[:, Hkv * D:2 * Hkv * D].unflatten(1, (Hkv, D))
+    out = prefill_attention(q, k, v, [40, 37], D ** -0.5)
+    want = prefill_attention(q, k.to(torch.float16).contiguous(), v.to(torch.float16).contiguous(), [40, 37], D ** -0.5)
+    assert torch.equal(out, want)
