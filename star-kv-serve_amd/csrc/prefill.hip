@@ -342,8 +342,7 @@ __global__ __launch_bounds__(PF_THR) __attribute__((amdgpu_waves_per_eu(2))) voi
 // ---------------------------------------------------------------------------
 // K and V of bf16 or fp32 as the fp16 rows that prefill_kernel reads: one launch, 8 values a
 // lane from rows at any strides, contiguous out. The bound is HBM (4 bytes read and written per
-// bf16 value). 16,384 tokens of 32 heads: 83 us where two
-// conversions of torch took 314.
+// bf16 value). 16,384 tokens of 32 heads: 83 us where two conversions of torch took 314.
 // ---------------------------------------------------------------------------
 struct ToHalfParams {
     const void* src[2]; int64_t s0[2], s1[2];  // elements: K, V
