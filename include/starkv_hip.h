@@ -424,6 +424,49 @@ int starkv_prefill_lift(void *stream, const void *k_codes, int64_t k_s0, const v
                         int v_rank);
 
 /*
+ * The decoder layer's operations around the attention (stock Llama in the reference,
+ * starkv_serve/model.py:77-106).
+ *
+ * starkv_rope_qkv: rotate-half RoPE of q [T, num_heads, 128] and, when given, k [T, num_kv_heads,
+ * 128] at positions [T] (int32 or int64; a negative one counts from the table's end, one outside
+ * it gives NaN) of cos_sin [cs_rows, 128] = cos | sin: fp32 arithmetic, rounded once to the inputs'
+ * dtype (bf16, fp16 or fp32). q_out and k_out are contiguous; k_cache / v_cache [num_blocks,
+ * block_size, num_kv_heads, 128] (shared element strides) take the rotated k and v at slot_mapping
+ * (a slot outside the cache: nothing); k_half / v_half [T, num_kv_heads, 128] take them in fp16.
+ * Every destination but q_out may be null. All rows 16-byte aligned.
+ *
+ * starkv_decode_slots: slots[b] = block_table[b][positions[b] / block_size] * block_size +
+ * positions[b] % block_size (-1 outside the row of `width` blocks) and seq_lens[b] = positions[b] + 1.
+ *
+ * starkv_greedy_step: tokens[b] = the index of the first largest of logits [n, width] (bf16, fp16 or
+ * fp32, rows 16-byte aligned; NaN counts as the largest), positions[b] += 1.
+ *
+ * starkv_silu_mul: out[t] = silu(gate_up[t, :width]) * gate_up[t, width:], silu rounded to the dtype
+ * before the product (bf16 or fp16, width a multiple of 8).
+ *
+ * starkv_few_linear: out [n, N] = x [n, K] w^T for the few tokens of a decode step (bf16 or fp16,
+ * fp32 sums, one rounding; starkv_few_linear_fits says whether n and K are taken). norm_weight [K]:
+ * x is first normalised (RMSNorm; bf16 only; h_out [n, K], when given, receives it rounded).
+ * mode 0: as it is; 1: plus residual [n, N] (no norm); 2: w [2 N, K] and silu(first N rows') *
+ * (the others') (with norm).
+ */
+int starkv_rope_qkv(void *stream, const void *q, int64_t q_s0, int64_t q_s1, const void *k, int64_t k_s0,
+                    int64_t k_s1, const void *v, int64_t v_s0, int64_t v_s1, int dtype, int num_tokens,
+                    int num_heads, int num_kv_heads, const void *positions, int pos_bits, const void *cos_sin,
+                    int64_t cs_s0, int cs_dtype, int64_t cs_rows, void *q_out, void *k_out, void *k_cache,
+                    void *v_cache, int64_t c_s0, int64_t c_s1, int64_t c_s2, int block_size, int64_t num_blocks,
+                    const void *slot_mapping, int slot_bits, void *k_half, void *v_half);
+int starkv_decode_slots(void *stream, const void *block_table, int64_t bt_s0, int64_t bt_s1, int bt_bits, int width,
+                        const int64_t *positions, int n, int block_size, int64_t *slots, int32_t *seq_lens);
+int starkv_greedy_step(void *stream, const void *logits, int64_t s0, int dtype, int n, int width, int64_t *tokens,
+                       int64_t *positions);
+int starkv_silu_mul(void *stream, const void *gate_up, int64_t s0, int dtype, int num_tokens, int width, void *out);
+int starkv_few_linear_fits(int n, int K);
+int starkv_few_linear(void *stream, const void *x, int64_t x_s0, const void *w, int64_t w_s0, int dtype, int n,
+                      int N, int K, const void *norm_weight, float eps, void *h_out, int mode, const void *residual,
+                      int64_t r_s0, void *out, int64_t o_s0);
+
+/*
  * Timing for benchmarks (no counterpart in the reference, whose benchmark reads profiler
  * traces instead, bench_serving.py:71-115). starkv_profile_begin arms up to max_calls
  * event pairs; each following decode call records one pair on its stream, around its

@@ -280,6 +280,116 @@ void prefill_lift(const at::Tensor& k_codes, const at::Tensor& v_codes, const at
           "prefill_lift");
 }
 
+const void* data_of(const std::optional<at::Tensor>& t) { return t ? t->data_ptr() : nullptr; }
+
+// RoPE of q (and k), with the cache write and the fp16 rows of an uncompressed layer; q, k, v
+// [T, heads, 128].
+void rope_qkv(const at::Tensor& q, const std::optional<at::Tensor>& k, const std::optional<at::Tensor>& v,
+              const at::Tensor& positions, const at::Tensor& cos_sin, const at::Tensor& q_out,
+              const std::optional<at::Tensor>& k_out, const std::optional<at::Tensor>& k_cache,
+              const std::optional<at::Tensor>& v_cache, const std::optional<at::Tensor>& slots,
+              const std::optional<at::Tensor>& k_half, const std::optional<at::Tensor>& v_half) {
+    const c10::DeviceGuard guard(q.device());
+    const int64_t T = q.size(0), H = q.size(1), Hkv = k ? k->size(1) : 0;
+    const auto rows = [&](const at::Tensor& t, int64_t heads) {
+        return t.dim() == 3 && t.size(0) == T && t.size(1) == heads && t.size(2) == 128 && t.stride(2) == 1;
+    };
+    TORCH_CHECK(rows(q, H) && rows(q_out, H) && q_out.is_contiguous() && q_out.scalar_type() == q.scalar_type(),
+                "starkv.rope_qkv: q");
+    for (const auto* t : {&k, &v})
+        TORCH_CHECK(!*t || (rows(**t, Hkv) && (*t)->scalar_type() == q.scalar_type()), "starkv.rope_qkv: k and v");
+    TORCH_CHECK(!k_out || (rows(*k_out, Hkv) && k_out->is_contiguous() && k_out->scalar_type() == q.scalar_type()),
+                "starkv.rope_qkv: k_out");
+    for (const auto* t : {&k_half, &v_half})
+        TORCH_CHECK(!*t || (rows(**t, Hkv) && (*t)->is_contiguous() && (*t)->scalar_type() == at::kHalf),
+                    "starkv.rope_qkv: fp16 rows");
+    TORCH_CHECK(positions.is_contiguous() && positions.numel() == T &&
+                    (positions.scalar_type() == at::kLong || positions.scalar_type() == at::kInt),
+                "starkv.rope_qkv: positions");
+    TORCH_CHECK(cos_sin.dim() == 2 && cos_sin.size(1) == 128 && cos_sin.stride(1) == 1, "starkv.rope_qkv: cos_sin");
+    if (k_cache)
+        TORCH_CHECK(v_cache && slots && slots->numel() >= T && k_cache->strides() == v_cache->strides() &&
+                        k_cache->sizes() == v_cache->sizes() && k_cache->size(2) == Hkv && k_cache->size(3) == 128 &&
+                        k_cache->stride(3) == 1 && k_cache->scalar_type() == q.scalar_type() &&
+                        v_cache->scalar_type() == q.scalar_type(),
+                    "starkv.rope_qkv: caches");
+    check(starkv_rope_qkv(stream_of(q), q.data_ptr(), q.stride(0), q.stride(1), data_of(k), k ? k->stride(0) : 0,
+                          k ? k->stride(1) : 0, data_of(v), v ? v->stride(0) : 0, v ? v->stride(1) : 0, dtype_code(q),
+                          (int)T, (int)H, (int)Hkv, positions.data_ptr(),
+                          positions.scalar_type() == at::kLong ? 64 : 32, cos_sin.data_ptr(), cos_sin.stride(0),
+                          dtype_code(cos_sin), cos_sin.size(0), q_out.data_ptr(), (void*)data_of(k_out),
+                          (void*)data_of(k_cache), (void*)data_of(v_cache), k_cache ? k_cache->stride(0) : 0,
+                          k_cache ? k_cache->stride(1) : 0, k_cache ? k_cache->stride(2) : 0,
+                          k_cache ? (int)k_cache->size(1) : 0, k_cache ? k_cache->size(0) : 0, data_of(slots),
+                          slots ? slot_bits(*slots) : 64, (void*)data_of(k_half), (void*)data_of(v_half)),
+          "rope_qkv");
+}
+
+// A decode step's slots (int64) and lengths (int32) from its positions (int64).
+void decode_slots(const at::Tensor& block_table, const at::Tensor& positions, int64_t block_size,
+                  const at::Tensor& slots, const at::Tensor& seq_lens) {
+    const c10::DeviceGuard guard(positions.device());
+    const int64_t n = positions.numel();
+    TORCH_CHECK(block_table.dim() == 2 && block_table.size(0) >= n &&
+                    (block_table.scalar_type() == at::kInt || block_table.scalar_type() == at::kLong) &&
+                    positions.is_contiguous() && positions.scalar_type() == at::kLong && slots.is_contiguous() &&
+                    slots.scalar_type() == at::kLong && slots.numel() == n && seq_lens.numel() == n,
+                "starkv.decode_slots: block_table [n, blocks], positions and slots [n] int64");
+    check(starkv_decode_slots(stream_of(positions), block_table.data_ptr(), block_table.stride(0), block_table.stride(1),
+                              block_table.scalar_type() == at::kInt ? 32 : 64, (int)block_table.size(1),
+                              positions.data_ptr<int64_t>(), (int)n, (int)block_size, slots.data_ptr<int64_t>(),
+                              (int32_t*)i32(seq_lens, "seq_lens")),
+          "decode_slots");
+}
+
+// tokens [n] = argmax of logits [n, vocab], positions [n] += 1 (int64).
+void greedy_step(const at::Tensor& logits, const at::Tensor& tokens, const at::Tensor& positions) {
+    const c10::DeviceGuard guard(logits.device());
+    TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1, "starkv.greedy_step: logits [n, vocab]");
+    for (const auto* t : {&tokens, &positions})
+        TORCH_CHECK(t->is_contiguous() && t->scalar_type() == at::kLong && t->numel() == logits.size(0),
+                    "starkv.greedy_step: tokens and positions [n] int64");
+    check(starkv_greedy_step(stream_of(logits), logits.data_ptr(), logits.stride(0), dtype_code(logits),
+                             (int)logits.size(0), (int)logits.size(1), tokens.data_ptr<int64_t>(),
+                             positions.data_ptr<int64_t>()),
+          "greedy_step");
+}
+
+// silu(gate) * up of gate_up [T, 2 width].
+void silu_mul(const at::Tensor& gate_up, const at::Tensor& out) {
+    const c10::DeviceGuard guard(gate_up.device());
+    TORCH_CHECK(gate_up.dim() == 2 && gate_up.stride(1) == 1 && out.is_contiguous() && out.dim() == 2 &&
+                    out.size(0) == gate_up.size(0) && 2 * out.size(1) == gate_up.size(1) &&
+                    out.scalar_type() == gate_up.scalar_type(),
+                "starkv.silu_mul: [T, 2 width] and [T, width]");
+    check(starkv_silu_mul(stream_of(gate_up), gate_up.data_ptr(), gate_up.stride(0), dtype_code(gate_up),
+                          (int)out.size(0), (int)out.size(1), out.data_ptr()),
+          "silu_mul");
+}
+
+// A weight product of a decode step's few tokens (mode: 0 plain, 1 plus residual, 2 gate).
+void few_linear(const at::Tensor& x, const at::Tensor& w, const std::optional<at::Tensor>& norm_weight, double eps,
+                const std::optional<at::Tensor>& h_out, int64_t mode, const std::optional<at::Tensor>& residual,
+                const at::Tensor& out) {
+    const c10::DeviceGuard guard(x.device());
+    const int64_t n = x.size(0), K = x.size(1), N = mode == 2 ? w.size(0) / 2 : w.size(0);
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == K && x.stride(1) == 1 && w.stride(1) == 1 &&
+                    w.scalar_type() == x.scalar_type() && (mode != 2 || w.size(0) % 2 == 0),
+                "starkv.few_linear: x [n, K] and w [N, K] of one dtype");
+    TORCH_CHECK(!norm_weight || (norm_weight->is_contiguous() && norm_weight->numel() == K &&
+                                 norm_weight->scalar_type() == x.scalar_type()),
+                "starkv.few_linear: norm weight");
+    TORCH_CHECK(!h_out || (h_out->is_contiguous() && h_out->sizes() == x.sizes() && h_out->scalar_type() == x.scalar_type()),
+                "starkv.few_linear: h_out");
+    for (const auto& t : {residual ? *residual : out, out})
+        TORCH_CHECK(t.dim() == 2 && t.size(0) == n && t.size(1) == N && t.stride(1) == 1 && t.scalar_type() == x.scalar_type(),
+                    "starkv.few_linear: out and residual [n, N]");
+    check(starkv_few_linear(stream_of(x), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), dtype_code(x), (int)n,
+                            (int)N, (int)K, data_of(norm_weight), (float)eps, (void*)data_of(h_out), (int)mode,
+                            data_of(residual), residual ? residual->stride(0) : 0, out.data_ptr(), out.stride(0)),
+          "few_linear");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(starkv, m) {
@@ -303,6 +413,15 @@ TORCH_LIBRARY(starkv, m) {
     m.def("stock_write(Tensor key, Tensor value, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping) -> ()");
     m.def("prefill(Tensor query, Tensor key, Tensor value, Tensor cu_seqlens, Tensor blocks, float scale, "
           "Tensor(a!) out) -> ()");
+    m.def("rope_qkv(Tensor q, Tensor? k, Tensor? v, Tensor positions, Tensor cos_sin, Tensor(a!) q_out, "
+          "Tensor(b!)? k_out, Tensor(c!)? k_cache, Tensor(d!)? v_cache, Tensor? slots, Tensor(e!)? k_half, "
+          "Tensor(f!)? v_half) -> ()");
+    m.def("decode_slots(Tensor block_table, Tensor positions, int block_size, Tensor(a!) slots, "
+          "Tensor(b!) seq_lens) -> ()");
+    m.def("greedy_step(Tensor logits, Tensor(a!) tokens, Tensor(b!) positions) -> ()");
+    m.def("silu_mul(Tensor gate_up, Tensor(a!) out) -> ()");
+    m.def("few_linear(Tensor x, Tensor w, Tensor? norm_weight, float eps, Tensor(a!)? h_out, int mode, "
+          "Tensor? residual, Tensor(b!) out) -> ()");
     m.def("prefill_to_half(Tensor key, Tensor value, Tensor(a!) key_out, Tensor(b!) value_out) -> ()");
     m.def("prefill_lift(Tensor k_codes, Tensor v_codes, Tensor cu_seqlens, Tensor k_up, Tensor k_offsets, "
           "Tensor k_widths, Tensor cos_sin, Tensor(a!) key, Tensor(b!)? v_out) -> ()");
@@ -318,6 +437,11 @@ TORCH_LIBRARY_IMPL(starkv, CUDA, m) {
     m.impl("stock_decode", &stock_decode);
     m.impl("stock_write", &stock_write);
     m.impl("prefill", &prefill);
+    m.impl("rope_qkv", &rope_qkv);
+    m.impl("decode_slots", &decode_slots);
+    m.impl("greedy_step", &greedy_step);
+    m.impl("silu_mul", &silu_mul);
+    m.impl("few_linear", &few_linear);
     m.impl("prefill_to_half", &prefill_to_half);
     m.impl("prefill_lift", &prefill_lift);
 }

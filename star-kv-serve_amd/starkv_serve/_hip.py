@@ -55,6 +55,13 @@ SIGNATURES = {
     "starkv_prefill_block_list": (_I, [ctypes.POINTER(ctypes.c_int32), _I, ctypes.POINTER(ctypes.c_int32), _I]),
     "starkv_prefill_attention": (_I, [_P, _P, _I64, _I64, _I, _P, _P, _I64, _I64, _I, _P, _P, _I, _I, _I, _I, _F,
                                       _P, _I64, _I64, _I]),
+    "starkv_rope_qkv": (_I, [_P, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _I, _I, _I, _I, _P, _I, _P, _I64, _I,
+                             _I64, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I64, _P, _I, _P, _P]),
+    "starkv_decode_slots": (_I, [_P, _P, _I64, _I64, _I, _I, _P, _I, _I, _P, _P]),
+    "starkv_greedy_step": (_I, [_P, _P, _I64, _I, _I, _I, _P, _P]),
+    "starkv_silu_mul": (_I, [_P, _P, _I64, _I, _I, _I, _P]),
+    "starkv_few_linear_fits": (_I, [_I, _I]),
+    "starkv_few_linear": (_I, [_P, _P, _I64, _P, _I64, _I, _I, _I, _I, _P, _F, _P, _I, _P, _I64, _P, _I64]),
     "starkv_prefill_to_half": (_I, [_P, _P, _I64, _I64, _P, _P, _I64, _I64, _P, _I, _I, _I]),
     "starkv_prefill_lift": (_I, [_P, _P, _I64, _P, _I64, _I, _I, _P, _I, _P, _I64, _P, _P, _I, _P, _I64, _I, _P,
                                  _P, _I]),

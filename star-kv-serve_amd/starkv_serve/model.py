@@ -36,6 +36,7 @@ import torch.nn.functional as F
 
 from starkv_serve.attention import StarKVAttentionImpl, StarKVMetadata
 from starkv_serve.checkpoint import StarKVCheckpoint
+from starkv_serve.kernels import model_ops
 from starkv_serve.kernels.prefill import prefill_attention
 from starkv_serve.kernels.stock_decode import paged_decode_full, write_kv_full
 from starkv_serve.workloads import cos_sin_table
@@ -56,6 +57,8 @@ class LlamaShape:
 
 LLAMA2_7B = LlamaShape()
 
+FEW_MAX_TOKENS = 16  # decode steps up to this many tokens take few_linear
+
 
 class Rotary:
     """What StarKVAttentionImpl reads of vLLM's RotaryEmbedding (``cos_sin_cache``
@@ -66,6 +69,8 @@ class Rotary:
 
     def apply(self, positions: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         """x [T, H, D] rotated at `positions` [T] (fp32 arithmetic, x's dtype out)."""
+        if model_ops.rope_fits(self.cos_sin_cache, positions, x):
+            return model_ops.rope(positions, x, self.cos_sin_cache)
         cos, sin = self.cos_sin_cache[positions].float().chunk(2, dim=-1)
         cos, sin = cos[:, None, :], sin[:, None, :]
         x1, x2 = x.float().chunk(2, dim=-1)
@@ -159,35 +164,79 @@ class StarKVLlamaForCausalLM:
                 self.kv_caches.append((kc, torch.zeros_like(kc)))
 
     # -- the step ---------------------------------------------------------------------------
-    def _attention(self, li: int, h: torch.Tensor, positions: torch.Tensor, md: StarKVMetadata,
-                   capture: Optional[list], in_graph: bool = False) -> torch.Tensor:
-        """Inside a graph (`in_graph`) no launch depends on the step's lengths: every layer
+    def _attention(self, li: int, x: torch.Tensor, positions: torch.Tensor, md: StarKVMetadata,
+                   capture: Optional[list], in_graph: bool, few: bool) -> torch.Tensor:
+        """The layer's attention from its residual stream x [T, hidden], up to o_proj's input.
+        Inside a graph (`in_graph`) no launch depends on the step's lengths: every layer
         decodes over the span max_model_len, the lengths are read on the device."""
         s, layer = self.shape, self.layers[li]
-        T = h.shape[0]
+        T = x.shape[0]
         H, Hkv, D = s.num_heads, s.num_kv_heads, s.head_dim
         k = v = None
         if layer.compressed:
-            q = self.rotary.apply(positions, F.linear(h, layer.q_proj).view(T, H, D))
+            h, q = self._norm_linear(x, layer.ln1, layer.q_proj, few, True)
+            q = self.rotary.apply(positions, q.view(T, H, D))
             out = torch.empty(T, H * D, dtype=self.dtype, device=self.device)
             layer.impl.forward_from_hidden(q.view(T, H * D), h, self.kv_caches[li], md, out, in_full_graph=in_graph)
         else:
-            qkv = F.linear(h, layer.qkv_proj)
-            q, k, v = qkv.split([H * D, Hkv * D, Hkv * D], dim=-1)
-            q = self.rotary.apply(positions, q.reshape(T, H, D))
-            k = self.rotary.apply(positions, k.reshape(T, Hkv, D))
-            v = v.reshape(T, Hkv, D)
+            h, qkv = self._norm_linear(x, layer.ln1, layer.qkv_proj, few, capture is not None)
+            q, k, v = (t.view(T, -1, D) for t in qkv.split([H * D, Hkv * D, Hkv * D], dim=-1))
             kc, vc = self.kv_caches[li]
-            write_kv_full(k, v, kc, vc, md.slot_mapping[:T])
+            ka, va = k, v  # the prefill attention's operands
+            if model_ops.rope_fits(self.rotary.cos_sin_cache, positions, q, k, v):
+                q, k, ka, va = model_ops.rope_write(positions, q, k, v, self.rotary.cos_sin_cache, kc, vc,
+                                                    md.slot_mapping[:T], capture is not None, bool(md.num_prefills))
+            else:
+                q, k = self.rotary.apply(positions, q), self.rotary.apply(positions, k)
+                ka = k
+                write_kv_full(k, v, kc, vc, md.slot_mapping[:T])
             if md.num_prefills:  # whole prompts only (prefill_step): causal attention over each prompt
-                out = prefill_attention(q, k, v, md.prefill_seq_lens_cpu, self.scale).view(T, H * D)
+                out = prefill_attention(q, ka, va, md.prefill_seq_lens_cpu, self.scale).view(T, H * D)
             else:
                 span = self.max_model_len if in_graph else max(md.max_seq_len, 1)
                 out = paged_decode_full(q, kc, vc, md.block_table[:T], md.seq_lens[:T], span,
                                         self.scale).view(T, H * D)
         if capture is not None:
             capture.append(dict(layer=li, q=q.view(T, H, D), out=out.view(T, H, D), h=h, k=k, v=v))
-        return F.linear(out, layer.o_proj)
+        return out
+
+    # -- the weight products ------------------------------------------------------------------
+    def _few(self, T: int, md: StarKVMetadata) -> bool:
+        """Whether this step's weight products run on ``few_linear``: a decode step of few tokens,
+        where the weights' bytes are the time. Llama-2-7B's widths at 16 tokens, us, against the
+        library's products with torch's norm, gate and sum: q 14 / 21, qkv 35 / 35, o 12 / 18, gate and
+        up 53 / 67, down 30 / 41, the head 74 / 68; the kernel's matrix tile holds 16 tokens."""
+        s = self.shape
+        return (self.device.type == "cuda" and not md.num_prefills and 1 <= T <= FEW_MAX_TOKENS
+                and self.dtype in (torch.bfloat16, torch.float16) and s.hidden_size % 32 == 0
+                and s.intermediate_size % 32 == 0)
+
+    def _norm_linear(self, x: torch.Tensor, ln: torch.Tensor, w: torch.Tensor, few: bool, want_h: bool) -> tuple:
+        """(the normalised x, when wanted, its product with w)."""
+        s = self.shape
+        if few and self.dtype == torch.bfloat16:
+            h = torch.empty_like(x) if want_h else None
+            return h, model_ops.few_linear(x, w, ln, s.rms_norm_eps, h)
+        h = F.rms_norm(x, (s.hidden_size,), ln, s.rms_norm_eps)
+        return h, model_ops.few_linear(h, w) if few else F.linear(h, w)
+
+    def _mlp(self, x: torch.Tensor, layer: Layer, few: bool) -> torch.Tensor:
+        """x plus the gated MLP of its norm."""
+        s = self.shape
+        if few and self.dtype == torch.bfloat16:
+            a = model_ops.few_linear(x, layer.gate_up, layer.ln2, s.rms_norm_eps, gate=True)
+        else:
+            gu = self._norm_linear(x, layer.ln2, layer.gate_up, few, False)[1]
+            if gu.is_cuda and gu.dtype in (torch.bfloat16, torch.float16) and s.intermediate_size % 8 == 0:
+                a = model_ops.silu_mul(gu)
+            else:
+                gate, up = gu.chunk(2, dim=-1)
+                a = F.silu(gate) * up
+        return self._add_linear(x, a, layer.down, few)
+
+    @staticmethod
+    def _add_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, few: bool) -> torch.Tensor:
+        return model_ops.few_linear(a, w, residual=x) if few else x + F.linear(a, w)
 
     @torch.no_grad()
     def attention_inputs(self, hidden: torch.Tensor, positions: torch.Tensor) -> List[tuple]:
@@ -232,25 +281,22 @@ class StarKVLlamaForCausalLM:
     @torch.no_grad()
     def _layers(self, x: torch.Tensor, positions: torch.Tensor, md: StarKVMetadata, capture: Optional[list],
                 in_graph: bool) -> torch.Tensor:
-        s = self.shape
+        few = self._few(x.shape[0], md)
         for li, layer in enumerate(self.layers):
-            h = F.rms_norm(x, (s.hidden_size,), layer.ln1, s.rms_norm_eps)
-            x = x + self._attention(li, h, positions, md, capture, in_graph)
-            h = F.rms_norm(x, (s.hidden_size,), layer.ln2, s.rms_norm_eps)
-            gate, up = F.linear(h, layer.gate_up).chunk(2, dim=-1)
-            x = x + F.linear(F.silu(gate) * up, layer.down)
+            x = self._add_linear(x, self._attention(li, x, positions, md, capture, in_graph, few), layer.o_proj, few)
+            x = self._mlp(x, layer, few)
         return x
 
-    def _logits(self, x: torch.Tensor) -> torch.Tensor:
-        s = self.shape
-        return F.linear(F.rms_norm(x, (s.hidden_size,), self.norm, s.rms_norm_eps), self.lm_head)
+    def _logits(self, x: torch.Tensor, few: bool) -> torch.Tensor:
+        return self._norm_linear(x, self.norm, self.lm_head, few, False)[1]
 
     def decode_step(self, tokens: torch.Tensor, positions: torch.Tensor, md: StarKVMetadata,
                     capture: Optional[list] = None, in_graph: bool = False) -> torch.Tensor:
         """Logits [n, vocab] for one new token per request: tokens [n] at `positions` [n];
         `md` has every row as a decode (seq_lens = positions + 1, slot_mapping the new
         tokens' slots)."""
-        return self._logits(self._layers(self.embed[tokens], positions, md, capture, in_graph))
+        x = self._layers(self.embed[tokens], positions, md, capture, in_graph)
+        return self._logits(x, self._few(x.shape[0], md))
 
     @torch.no_grad()
     def prefill_step(self, tokens: torch.Tensor, positions: torch.Tensor, md: StarKVMetadata,
@@ -263,7 +309,7 @@ class StarKVLlamaForCausalLM:
             raise ValueError("prefill_step: a prompts-only batch (prefill_metadata)")
         x = self._layers(self.embed[tokens], positions, md, capture, False)
         last = torch.tensor(md.prefill_query_start_loc_cpu[1:], device=x.device) - 1
-        return self._logits(x[last])
+        return self._logits(x[last], False)
 
 
 class DecodeGraph:
@@ -294,8 +340,11 @@ class DecodeGraph:
         m = self.model
         md = decode_metadata(self.block_table, self.positions, m.block_size, m.max_model_len)
         self.logits = m.decode_step(self.tokens, self.positions, md, in_graph=True)
-        self.tokens.copy_(self.logits.argmax(-1))
-        self.positions.add_(1)
+        if self.tokens.dtype == torch.int64 and m.shape.vocab_size % 8 == 0:
+            model_ops.greedy_step(self.logits, self.tokens, self.positions)
+        else:
+            self.tokens.copy_(self.logits.argmax(-1))
+            self.positions.add_(1)
 
     def reset(self, tokens: torch.Tensor, positions: torch.Tensor) -> None:
         self.tokens.copy_(tokens)
@@ -313,11 +362,16 @@ def decode_metadata(block_table: torch.Tensor, positions: torch.Tensor, block_si
     if max_seq_len > block_table.shape[1] * block_size:
         raise ValueError(f"positions up to {max_seq_len - 1} need more than the block table's "
                          f"{block_table.shape[1]} blocks of {block_size}")
-    rows = torch.arange(n, device=positions.device)
-    slots = block_table[rows, positions // block_size].long() * block_size + positions % block_size
+    if (positions.is_cuda and block_table.device == positions.device and positions.dtype == torch.int64
+            and positions.is_contiguous() and block_table.dtype in (torch.int32, torch.int64)
+            and block_table.shape[0] >= n):
+        slots, seq_lens = model_ops.decode_slots(block_table, positions, block_size)
+    else:
+        rows = torch.arange(n, device=positions.device)
+        slots = block_table[rows, positions // block_size].long() * block_size + positions % block_size
+        seq_lens = (positions + 1).to(torch.int32)
     return StarKVMetadata(num_actual_tokens=n, num_decodes=n, num_decode_tokens=n, num_prefills=0,
-                          max_seq_len=int(max_seq_len), seq_lens=(positions + 1).to(torch.int32),
-                          block_table=block_table, slot_mapping=slots)
+                          max_seq_len=int(max_seq_len), seq_lens=seq_lens, block_table=block_table, slot_mapping=slots)
 
 
 def prefill_metadata(block_table: torch.Tensor, prompt_lens: List[int], block_size: int):
