@@ -423,9 +423,8 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
 //   column's weighted sum of their accumulators, U partials' loads in flight, divided by the
 //   total, into o [n][Hq][ld] (NaN for a request with no tokens, as the reference's softmax
 //   over an empty row). MCW = 1: the four waves take different columns (1024 per
-//   workgroup), each over every slot; MCW = 8 (eight waves), for requests split over many
-//   workgroups (a few long requests): wave w sums slots w, w + 8, ... of 256 columns, then
-//   the waves' sums are added.
+//   workgroup), each over every slot; MCW = 4, for requests split over many workgroups:
+//   wave w sums slots w, w + 4, ... of 256 columns, then the waves' sums are added.
 // lift_kernel<DT, REQ, THR, DQ>: one workgroup per (head, REQ requests, 8 DQ output
 //   columns): out = o @ v_up_by_q[h], each thread 8 output columns over a THR / DQ-th of the
 //   rank columns, LIFT_U rows in flight, then a reduction over those parts. 8 requests x
@@ -441,6 +440,7 @@ template <int MCW, int U, int THR>
 __global__ __launch_bounds__(THR) void merge_cols_kernel(const uint8_t* __restrict__ ws, size_t ws_plan, size_t ws_m,
                                                             size_t ws_l, size_t ws_acc, size_t ws_o, int n, int Hq,
                                                             int v_rank, int ld, int pv_r) {
+    static_assert(MCW == 1 || THR == 64 * MCW, "a wave a phase, or every wave its own columns");
     constexpr int CPW = 4 * THR / MCW;  // columns per workgroup
     __shared__ f32x4_t s_sum[MCW][64];
     __shared__ float s_mr[64 * MC_WREG];  // R > 1: the slots' maxima held in registers, for reads by index
@@ -653,6 +653,134 @@ __global__ __launch_bounds__(LIFT_THR) void lift_kernel(const uint8_t* __restric
     }
 }
 
+// lift_matrix_kernel<RT>: the lift of bf16 v_up_by_q on v_mfma_f32_16x16x32_bf16. One workgroup of 8
+// waves per (head, 16 RT requests, 32 output columns), the rank columns split over the waves, six
+// steps of 32 of them in flight. A = v_up^T: a step's 32 rows x 64 bytes go through the wave's own
+// LDS and come back transposed (ds_read_b64_tr_b16); B = the rows o as three bf16 values each (8 + 8
+// + 8 bits hold an fp32 value exactly, so the products are those of fp32 o and their sums fp32: no
+// less precise than fmaf, where an inf or NaN takes the first value only). The vector form spends 8
+// fmaf and an LDS read per 8 columns and request. LIFT_FIGURES
+constexpr int LM_WAVES = 8;
+constexpr int LM_BATCH = 6;  // steps of 32 rank columns in flight per wave
+constexpr int LM_LDS = LM_WAVES * LM_BATCH * 2048;
+
+template <int RT>
+__global__ __launch_bounds__(64 * LM_WAVES) void lift_matrix_kernel(const uint8_t* __restrict__ ws, size_t ws_o, int n, int Hq,
+                                                                    int v_rank, int ld, const uint16_t* __restrict__ vup,
+                                                                    int64_t vu_s0, int64_t vu_s1, void* __restrict__ out,
+                                                                    int64_t o_s0, int64_t o_s1, int out_dt) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __align__(16) uint8_t s_dyn[];
+    const int h = blockIdx.x, b0 = blockIdx.y * 16 * RT, d0 = blockIdx.z * 32;
+    const int tid = threadIdx.x, lane = tid & 63, w = rfl(tid >> 6), g = lane >> 4, li = lane & 15;
+    uint8_t* mine = s_dyn + w * LM_BATCH * 2048;
+    const uint32_t lds = lds_addr(mine);
+    const int steps = (v_rank + 31) >> 5, s0 = steps * w / LM_WAVES, s1 = steps * (w + 1) / LM_WAVES;
+    const uint16_t* vu = vup + (int64_t)h * vu_s0 + d0 + 8 * (lane & 3);
+    const float* orow[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+        orow[t] = (const float*)(ws + ws_o) + ((int64_t)min(b0 + 16 * t + li, n - 1) * Hq + h) * ld;
+    // Row r of a step (64 bytes) at 64 r, its halves exchanged in every second run of 8 rows: the
+    // four 16-lane groups of a transposing read take rows 8 g .. of the same half.
+    const uint32_t put = (uint32_t)((lane >> 2) * 64 + 16 * ((lane & 3) ^ (((lane >> 5) & 1) << 1)));
+    uint32_t get[2][2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int row = 8 * g + 4 * t + (li >> 2);
+            get[c][t] = lds + (uint32_t)(row * 64 + 32 * (c ^ (g & 1)) + 8 * (li & 3));
+        }
+    f32x4_t acc[RT][2];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[t][c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += LM_BATCH) {
+        u4 a[LM_BATCH][2];
+        f32x4_t x[LM_BATCH][RT][2];
+#pragma unroll
+        for (int i = 0; i < LM_BATCH; ++i) {
+            const int st = min(s + i, s1 - 1);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int r = 32 * st + 16 * j + (lane >> 2);
+                a[i][j] = *(const u4*)(vu + (int64_t)min(r, v_rank - 1) * vu_s1);
+                if (r >= v_rank) a[i][j] = (u4){0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {  // ld is v_rank rounded up to 4: whole or past the row
+                    const int k = 32 * st + 8 * g + 4 * j;
+                    x[i][t][j] = *(const f32x4_t*)(orow[t] + min(k, ld - 4));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (k + e >= v_rank) x[i][t][j][e] = 0.f;
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < LM_BATCH; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) *(u4*)(mine + i * 2048 + j * 1024 + put) = a[i][j];
+#pragma unroll
+        for (int i = 0; i < LM_BATCH; ++i) {
+            if (s + i >= s1) break;
+            bf16x8_t va[2];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const uint2 p = tr_read(get[c][0] + 2048 * i), q = tr_read(get[c][1] + 2048 * i);
+                va[c] = __builtin_bit_cast(bf16x8_t, make_uint4(p.x, p.y, q.x, q.y));
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                uint32_t part[3][4];  // the three values of 8 columns, two a word
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    uint32_t b[2][3];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const float v = x[i][t][(e + k) >> 2][(e + k) & 3];
+                        const bool fin = fabsf(v) < INFINITY;
+                        b[k][0] = __float_as_uint(v) & 0xffff0000u;
+                        const float r1 = fin ? v - __uint_as_float(b[k][0]) : 0.f;
+                        b[k][1] = __float_as_uint(r1) & 0xffff0000u;
+                        b[k][2] = __float_as_uint(r1 - __uint_as_float(b[k][1]));
+                    }
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) part[q][e >> 1] = (b[0][q] >> 16) | (b[1][q] & 0xffff0000u);
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const bf16x8_t ob = __builtin_bit_cast(bf16x8_t, make_uint4(part[q][0], part[q][1], part[q][2], part[q][3]));
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+                        acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[c], ob, acc[t][c], 0, 0, 0);
+                }
+            }
+        }
+    }
+    // The waves' sums: entry (wave, request tile, column tile, lane), over the rows' LDS.
+    __syncthreads();
+    f32x4_t* sum = (f32x4_t*)s_dyn;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sum[((w * RT + t) * 2 + c) * 64 + lane] = acc[t][c];
+    __syncthreads();
+    // Column 16 c + 4 (l / 16) + e of request l % 16 is element e of lane l.
+    for (int i = tid; i < RT * 512; i += 64 * LM_WAVES) {
+        const int t = i >> 9, col = i & 31, r = (i >> 5) & 15, b = b0 + 16 * t + r;
+        if (b >= n) continue;
+        float v = 0.f;
+#pragma unroll
+        for (int k = 0; k < LM_WAVES; ++k)
+            v += ((const float*)&sum[((k * RT + t) * 2 + (col >> 4)) * 64 + 16 * ((col >> 2) & 3) + r])[col & 3];
+        store_f(out, (int64_t)b * o_s0 + (int64_t)h * o_s1 + d0 + col, out_dt, v);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Host side of the P @ V pass and the merge.
 // ---------------------------------------------------------------------------
@@ -807,17 +935,32 @@ int launch_merge_wide(const DecodeParams& p, int grid, int w_dt, const void* vup
                       void* out, int64_t o_s0, int64_t o_s1, int out_dt, hipStream_t stream) {
     const size_t lds = lift_lds(p.acc_ld);
     SKV_CHECK(lds <= (size_t)PV_MAX_DYN_LDS, "decode: v_rank %d too large for the merge", p.v_rank);
-    // Slots per request: about gp / n + 1. Many (a few long requests): split them over waves.
+    // Partials per request: about gp / n + 1, many of them split over the waves. Whole decode at W 880,
+    // r_v 1280, us, with 16, 4 and 1 waves' phases: 1 request of 16384 tokens 65.7, 62.5, 72.6; 2 of 8192
+    // 65.9, 62.5, 64.6; 8 of 4096 84.7, 80.6, 79.8; 24 179.5, 162.6, 159.7; 48 310, 263, 259.
     const int gp = (grid + p.pv_r - 1) / p.pv_r;
-    if (gp >= 8 * p.n)
-        hipLaunchKernelGGL((merge_cols_kernel<16, 8, 1024>), dim3(p.n, p.Hq, (p.v_rank + 255) / 256), dim3(1024), 0,
-                           stream, (const uint8_t*)p.ws, p.ws_plan, p.ws_m, p.ws_l, p.ws_acc, p.ws_o, p.n, p.Hq,
-                           p.v_rank, p.acc_ld, p.pv_r);
-    else
-        hipLaunchKernelGGL((merge_cols_kernel<1, 8, MC_THR>), dim3(p.n, p.Hq, (p.v_rank + 1023) / 1024), dim3(MC_THR), 0,
-                           stream, (const uint8_t*)p.ws, p.ws_plan, p.ws_m, p.ws_l, p.ws_acc, p.ws_o, p.n, p.Hq,
-                           p.v_rank, p.acc_ld, p.pv_r);
-    SKV_HIP(hipGetLastError());
+    const int waves = gp >= 48 * p.n ? 4 : 1;
+    const void* mc = waves == 4 ? (const void*)&merge_cols_kernel<4, 8, MC_THR> : (const void*)&merge_cols_kernel<1, 8, MC_THR>;
+    const uint8_t* ws = p.ws;
+    size_t wplan = p.ws_plan, wm = p.ws_m, wl = p.ws_l, wa = p.ws_acc, wo = p.ws_o;
+    int n = p.n, Hq = p.Hq, vr = p.v_rank, ld = p.acc_ld, pvr = p.pv_r;
+    void* margs[] = {(void*)&ws, (void*)&wplan, (void*)&wm, (void*)&wl, (void*)&wa, (void*)&wo,
+                     (void*)&n, (void*)&Hq, (void*)&vr, (void*)&ld, (void*)&pvr};
+    const int cols = 4 * MC_THR / waves;
+    SKV_HIP(hipLaunchKernel(mc, dim3(n, Hq, (vr + cols - 1) / cols), dim3(MC_THR), margs, 0, stream));
+    // Up to 4 requests the vector form's 128 workgroups a request pair are as quick (W 880, r_v 1280,
+    // whole decode, us, vector / matrix: 1 request 64.7 / 64.6, 4 77.6 / 77.8, 8 81.2 / 75.5). fp16 rows
+    // stay with it: an fp32 sum in fp16 parts would lose its small values.
+    const bool matrix = n > 4 && w_dt == STARKV_BF16 && (uintptr_t)vup % 16 == 0 && vu_s0 % 8 == 0 && vu_s1 % 8 == 0;
+    if (matrix) {
+        const int rt = n > 16 ? 2 : 1;
+        const void* fm = rt == 2 ? (const void*)&lift_matrix_kernel<2> : (const void*)&lift_matrix_kernel<1>;
+        if (int rc = raise_lds(fm, LM_LDS)) return rc;
+        void* largs[] = {(void*)&ws, (void*)&wo, (void*)&n, (void*)&Hq, (void*)&vr, (void*)&ld, (void*)&vup,
+                         (void*)&vu_s0, (void*)&vu_s1, (void*)&out, (void*)&o_s0, (void*)&o_s1, (void*)&out_dt};
+        SKV_HIP(hipLaunchKernel(fm, dim3(Hq, (n + 16 * rt - 1) / (16 * rt), 4), dim3(64 * LM_WAVES), largs, LM_LDS, stream));
+        return STARKV_OK;
+    }
     const bool small = p.n <= 8;
     const int req = small ? 2 : 8, thr = small ? 1024 : 512, dq = small ? 4 : 16;
     const void* fn = small ? (w_dt == STARKV_BF16 ? (const void*)&lift_kernel<STARKV_BF16, 2, 1024, 4>
@@ -830,9 +973,6 @@ int launch_merge_wide(const DecodeParams& p, int grid, int w_dt, const void* vup
     if (rc) return rc;
     const size_t lds2 = lift_lds(p.acc_ld, req, thr, dq);
     SKV_CHECK(lds2 <= (size_t)PV_MAX_DYN_LDS, "decode: v_rank %d too large for the lift", p.v_rank);
-    const uint8_t* ws = p.ws;
-    size_t wo = p.ws_o;
-    int n = p.n, Hq = p.Hq, vr = p.v_rank, ld = p.acc_ld;
     void* args[] = {(void*)&ws, (void*)&wo, (void*)&n, (void*)&Hq, (void*)&vr, (void*)&ld, (void*)&vup,
                     (void*)&vu_s0, (void*)&vu_s1, (void*)&out, (void*)&o_s0, (void*)&o_s1, (void*)&out_dt};
     SKV_HIP(hipLaunchKernel(fn, dim3(p.Hq, (p.n + req - 1) / req, 128 / (8 * dq)), dim3(thr), args, lds2, stream));

@@ -557,3 +557,33 @@ def test_k_up_and_v_up_dtypes_independent(cuda):
     out = paged_starkv_decode(*g.decode_args())
     assert out.dtype == torch.float32
     assert_close(out.to(torch.bfloat16), truth, "k_up bf16, v_up fp32")
+
+
+@pytest.mark.parametrize("n,v_rank,quant", [(5, 1280, False), (16, 1290, True), (17, 264, False), (33, 1283, True)])
+def test_two_pass_lift_on_matrix_instructions(cuda, n, v_rank, quant):
+    """More than four requests' lift of bf16 v_up_by_q: request counts around the tile of 16, rank
+    columns that are no multiple of a step of 32 or of a batch, one request without tokens (NaN,
+    as the softmax over an empty row) beside the others. fp32 output against the vector form's
+    (fp16 v_up_by_q of the same values, which bf16 holds exactly): the same products, sums of
+    v_rank terms in another order."""
+    lens = [0] + [17 + 29 * i for i in range(n - 1)]
+    kw = dict(num_heads=8, seed=n, v_rank=v_rank)
+    wl = (W.make_quant if quant else W.make_lowrank)(lens, **kw)
+    g = wl.to(cuda)
+    args = list(g.decode_args())
+    at = [i for i, a in enumerate(args) if torch.is_tensor(a) and a.data_ptr() == g.v_up_by_q.data_ptr()][0]
+    fn = paged_quant_decode if quant else paged_starkv_decode
+    v16 = g.v_up_by_q.to(torch.bfloat16).to(torch.float16)  # values both dtypes hold
+    outs = []
+    for dt in (torch.bfloat16, torch.float16):
+        args[at] = v16.to(dt)
+        out = torch.empty(n, 8, 128, dtype=torch.float32, device=cuda)
+        fn(*args, out=out)
+        outs.append(out.double())
+    assert torch.equal(v16.to(torch.bfloat16).double(), v16.double())
+    assert outs[0][0].isnan().all() and outs[1][0].isnan().all()
+    a, b = outs[0][1:], outs[1][1:]
+    assert torch.isfinite(a).all()
+    # Averages of normal codes: |o| <= 8. Two fp32 sums of v_rank products each.
+    bound = 2 * v_rank * 2.0 ** -24 * 8 * v16.double().abs().sum(1).max()
+    assert ((a - b).abs() <= bound).all()
