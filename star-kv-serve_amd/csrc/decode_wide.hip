@@ -48,7 +48,7 @@ namespace starkv {
 
 namespace {
 
-constexpr int PV_MAX_DYN_LDS = 160 * 1024 - 1024;  // the kernel's static LDS is a few words
+constexpr int PV_MAX_DYN_LDS = 160 * 1024 - 4096;  // beside at most 4 KB of P
 
 // Swizzled slot of token t in granule column G.
 __device__ __forceinline__ int gslot(int G, int t) { return t ^ ((G & 1) << 2); }
@@ -60,20 +60,6 @@ typedef __attribute__((address_space(3))) short4v_t* lds_s4p;
 __device__ __forceinline__ uint2 tr_read(uint32_t addr) {
     const short4v_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4p)(uintptr_t)addr);
     return __builtin_bit_cast(uint2, r);
-}
-
-// Packs 8 fp32 values into 8 bfloat16 (round to nearest even).
-__device__ __forceinline__ bf16x8_t to_bf16x8(const float (&v)[8]) {
-    bf16x8_t r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (__bf16)v[e];
-    return r;
-}
-__device__ __forceinline__ half8_t to_f16x8(const float (&v)[8]) {
-    half8_t r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = (_Float16)v[e];
-    return r;
 }
 
 }  // namespace
@@ -105,21 +91,22 @@ struct PvParams {
 };
 
 
-// Copy descriptors of one page (record r; valid false past the range: nothing is read):
-// its rows, its logits (request b, tokens 16 k .., every head), the reference maxima of the
-// R logits-pass slots b + R g + j.
+// Copy descriptors: the rows of one page (record r) and, of the page after it (record rn), the
+// logits (request b, tokens 16 k .., every head) and the reference maxima of the R logits-pass
+// slots b + R g + j. Past the range (v, vn false) nothing is read.
 struct PvPage {
     int4v_t rv, rl, rm;
 };
 
-__device__ __forceinline__ PvPage pv_page_desc(const PvParams& p, const PageRec& r, bool v, int g) {
+__device__ __forceinline__ PvPage pv_page_desc(const PvParams& p, const PageRec& r, bool v, const PageRec& rn, bool vn,
+                                               int g) {
     PvPage d;
-    const int b = v ? pr_b(r.bits) : 0, k = v ? r.k : 0;
     d.rv = buffer_rsrc((const void*)(uintptr_t)r.addr, v ? pr_rows(r.bits) * p.c_s1 : 0);
+    const int b = vn ? pr_b(rn.bits) : 0, k = vn ? rn.k : 0;
     const uint8_t* lg = p.ws + p.ws_lg + (((int64_t)b * (p.lcap / TILE_TOK) + k) * p.Hq * TILE_TOK) * 4;
-    d.rl = buffer_rsrc(lg, v ? p.Hq * TILE_TOK * 4 : 0);
+    d.rl = buffer_rsrc(lg, vn ? p.Hq * TILE_TOK * 4 : 0);
     const uint8_t* m = p.ws + p.ws_m + (int64_t)(b + p.r * g) * p.Hq * 4;
-    d.rm = buffer_rsrc(m, v ? ((p.r * p.Hq * 4 + 15) & ~15) : 0);
+    d.rm = buffer_rsrc(m, vn ? ((p.r * p.Hq * 4 + 15) & ~15) : 0);
     return d;
 }
 
@@ -132,20 +119,20 @@ __device__ __forceinline__ PageRec pv_rec(const PvParams& p, int j) {
 // columns.
 constexpr int PV_V0 = 3;
 
-// The copies of this wave for one page into the buffer at LDS byte `buf`: copy i moves
-// chunk 8 i + wave; chunks past nch go to the dummy block and read nothing.
+// The copies of this wave for one page's V (descriptor rv) into the buffer at LDS byte `buf`
+// and the logits and maxima of the page after it (rl, rm) into the buffer at `lbuf`: copy i
+// moves chunk 8 i + wave; chunks past nch go to the dummy block and read nothing.
 template <int NLD>
-__device__ __forceinline__ void pv_copies(const PvParams& p, const PvPage& d, uint32_t buf, uint32_t dummy, int wave,
-                                          const uint32_t (&off)[NLD]) {
+__device__ __forceinline__ void pv_copies(const PvParams& p, const PvPage& d, uint32_t buf, uint32_t lbuf, uint32_t dummy,
+                                          int wave, const uint32_t (&off)[NLD]) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         if (i >= p.nld) break;
         const int ch = i * NWAVE + wave;
-        const uint32_t m0 = ch < p.nch ? buf + (uint32_t)ch * 1024u : dummy;
         if (i == 0 && wave < PV_V0)
-            lds_copy16(wave < 2 ? d.rl : d.rm, m0, off[i]);
+            lds_copy16(wave < 2 ? d.rl : d.rm, lbuf + (uint32_t)ch * 1024u, off[i]);
         else
-            lds_copy16(d.rv, m0, off[i]);
+            lds_copy16(d.rv, ch < p.nch ? buf + (uint32_t)ch * 1024u : dummy, off[i]);
     }
 }
 
@@ -167,6 +154,9 @@ __device__ __forceinline__ half2_t nib2(uint32_t w, uint32_t sel) {
 template <int FMT, int MB, int NLD, bool MULTI>
 __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_pv[];
+    // P of the current and the next page as the MFMA's A operand: [page parity][bf16: high and
+    // low parts][lane][8].
+    __shared__ __attribute__((aligned(16))) uint16_t s_p[2][FMT == FMT_BF16 ? 2 : 1][64][8];
     // The parameters by value: the page loop's fields stay in registers (this kernel has
     // the registers to spare) instead of being reloaded where they are used.
     const PvParams& p = p0;
@@ -211,8 +201,8 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
         off[i] = o;
     }
 
-    // A operand: head am = lane & 31, tokens 8 ag .. 8 ag + 7 (ag = lane >> 5).
-    const int am = lane & 31, ag = lane >> 5;
+    // A operand: head lane & 31, tokens 8 ag .. 8 ag + 7.
+    const int ag = lane >> 5;
     // B operand reads of block (or chunk) 0, relative to the page buffer.
     uint32_t trd0, trd1;
     {
@@ -231,25 +221,37 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
             trd1 = (uint32_t)((G * 16 + gslot(G, t + 4)) * 16 + 8 * h);
         }
     }
-    const uint32_t lga = (uint32_t)((am * 16 + 8 * ag) * 4);  // logits of (am, 8 ag ..)
-    const uint32_t mxa = (uint32_t)(2 * 1024 + am * 4);         // slot 0's max of head am
+    // Forming P: this lane's head ph and token pt of a page; logits and slot 0's max of it in a page
+    // buffer, its place in s_p (operand lane ph + 32 (pt / 8), element pt % 8).
+    const int ph = 4 * wave + (lane >> 4), pt = lane & 15;
+    const uint32_t lga = (uint32_t)((ph * 16 + pt) * 4), mxa = (uint32_t)(2 * 1024 + ph * 4);
+    uint16_t* pput = &s_p[0][0][ph + 32 * (pt >> 3)][pt & 7];
     __syncthreads();
 
     f32x16_t acc[MB];
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[i] = (f32x16_t){};
 
-    // Records: the current page j (cur), j + 1 (ncur, loaded in iteration j), the page whose
-    // copies issue in iteration j (cpy = page j + nbuf - 1, loaded in iteration j - 1).
-    PageRec cur = pv_rec(p, beg);
-    // Prologue: pages beg .. beg + nbuf - 2 in flight.
-    for (int j = 0; j < p.nbuf - 1; ++j) {
-        const bool v = beg + j < end;
-        const PageRec r = v ? pv_rec(p, beg + j) : cur;
-        pv_copies<NLD>(p, pv_page_desc(p, r, v, g), base + (uint32_t)(j * p.buf_bytes), dummy, wave, off);
+    // Records: the current page j (cur) and the next (nxt); the page whose V copies issue in
+    // iteration j (cpy = page j + nbuf - 1) and the one after it, whose logits do (cpl). Each is
+    // loaded an iteration before its use.
+    PageRec cur = pv_rec(p, beg), nxt = beg + 1 < end ? pv_rec(p, beg + 1) : cur;
+    // Prologue: the logits of page beg, then V of pages beg .. beg + nbuf - 2, each with the next
+    // page's logits, in flight.
+    if (wave < PV_V0) {
+        const PvPage d = pv_page_desc(p, cur, false, cur, true, g);
+        lds_copy16(wave < 2 ? d.rl : d.rm, base + (uint32_t)wave * 1024u, off[0]);
     }
-    int jc = beg + p.nbuf - 1;  // the page whose copies issue next
-    PageRec cpy = jc < end ? pv_rec(p, jc) : cur;
+    PageRec cpy = cur;
+    for (int j = 0; j < p.nbuf - 1; ++j) {
+        const bool v = beg + j < end, vn = beg + j + 1 < end;
+        const PageRec rn = vn ? pv_rec(p, beg + j + 1) : cur;
+        pv_copies<NLD>(p, pv_page_desc(p, cpy, v, rn, vn, g), base + (uint32_t)(j * p.buf_bytes),
+                       base + (uint32_t)((j + 1) * p.buf_bytes), dummy, wave, off);
+        cpy = rn;
+    }
+    int jc = beg + p.nbuf - 1;  // the page whose V copies issue next
+    PageRec cpl = jc + 1 < end ? pv_rec(p, jc + 1) : cur;
     int jb = 0;  // buffer of the current page
     // The logits-pass ranges R g + j holding pages of request b: bit j. This pass's
     // reference max of the request is the largest of theirs (slots of other ranges hold
@@ -264,25 +266,9 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
         }
         return msk;
     };
-    int msk = sub_mask(pr_b(cur.bits));  // of the current request, redone when the request changes
-    for (int j = beg; j < end; ++j) {
-        // Page j is in buffer jb; the copies of the nbuf - 2 pages after it may still run.
-        wait_vmcnt_lgkm0_wide((p.nbuf - 2) * p.nld);
-        wait_lgkm0_barrier();  // every wave is done with the previous page's buffer
-        {
-            const int jn = jb == 0 ? p.nbuf - 1 : jb - 1;  // the buffer the previous page used
-            pv_copies<NLD>(p, pv_page_desc(p, cpy, jc < end, g), base + (uint32_t)(jn * p.buf_bytes), dummy, wave,
-                           off);
-        }
-        // The records of the next iteration: they arrive under its wait.
-        ++jc;
-        const PageRec ncpy = jc < end ? pv_rec(p, jc) : cur;
-        const PageRec ncur = j + 1 < end ? pv_rec(p, j + 1) : cur;
-        const int rows = pr_rows(cur.bits);
-        const uint32_t buf = base + (uint32_t)(jb * p.buf_bytes);
-        const uint32_t vbuf = buf + PV_V0 * 1024;  // the page's V granule columns
-        // A operand: P of head am at tokens 8 ag .. 8 ag + 7 of this page.
-        const f32x4_t s0 = lds_ld<f32x4_t>(buf + lga), s1 = lds_ld<f32x4_t>(buf + lga + 16);
+    int msk = sub_mask(pr_b(cur.bits));  // of the next page's request, redone when the request changes
+    // P of a page (its record r, its logits in the buffer at lbuf) into s_p[par]: one value a lane.
+    auto form_p = [&](const PageRec& r, uint32_t lbuf, int par) {
         // R = 1: the slot's max. Else the largest of the R slots' maxima (all four read:
         // the slots past R are in the chunk too), those of other requests' ranges left out.
         float mx;
@@ -290,25 +276,50 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
             mx = -INFINITY;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float mj = lds_ld<float>(buf + mxa + (uint32_t)(4 * j * p.Hq));
+                const float mj = lds_ld<float>(lbuf + mxa + (uint32_t)(4 * j * p.Hq));
                 mx = (msk >> j) & 1 ? fmaxf(mx, mj) : mx;
             }
         } else {
-            mx = lds_ld<float>(buf + mxa);
+            mx = lds_ld<float>(lbuf + mxa);
         }
-        const float sv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
-        const int tok0 = 8 * ag;  // this lane's first token in the page
-        float pe[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool ok = am < p.Hq && tok0 + e < rows;
-            pe[e] = __builtin_amdgcn_exp2f(ok ? sv[e] - mx : -INFINITY);  // no branch: exp2(-inf) = 0
-        }
+        const bool ok = ph < p.Hq && pt < pr_rows(r.bits);
+        const float pe = __builtin_amdgcn_exp2f(ok ? lds_ld<float>(lbuf + lga) - mx : -INFINITY);  // exp2(-inf) = 0
+        uint16_t* at = pput + par * (int)(sizeof(s_p[0]) / 2);
         if constexpr (FMT == FMT_BF16) {
-            float lo[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) lo[e] = pe[e] - (float)(__bf16)pe[e];
-            const bf16x8_t ahi = to_bf16x8(pe), alo = to_bf16x8(lo);
+            const __bf16 hi = (__bf16)pe;
+            at[0] = __builtin_bit_cast(uint16_t, hi);
+            at[64 * 8] = __builtin_bit_cast(uint16_t, (__bf16)(pe - (float)hi));
+        } else {
+            at[0] = __builtin_bit_cast(uint16_t, (_Float16)pe);
+        }
+    };
+    wait_vmcnt_lgkm0_wide((p.nbuf - 1) * p.nld);  // page beg's logits have landed
+    wait_lgkm0_barrier();
+    form_p(cur, base, 0);
+    if (MULTI && beg + 1 < end) msk = sub_mask(pr_b(nxt.bits));
+    for (int j = beg; j < end; ++j) {
+        // Page j's V is in buffer jb and page j + 1's logits in the next; the copies of the
+        // nbuf - 2 pages after them may still run.
+        wait_vmcnt_lgkm0_wide((p.nbuf - 2) * p.nld);
+        wait_lgkm0_barrier();  // every wave is done with the previous page's buffer, P of page j is whole
+        const uint32_t buf = base + (uint32_t)(jb * p.buf_bytes);
+        {
+            const int jn = jb == 0 ? p.nbuf - 1 : jb - 1;  // the buffer whose V the previous page used
+            pv_copies<NLD>(p, pv_page_desc(p, cpy, jc < end, cpl, jc + 1 < end, g), base + (uint32_t)(jn * p.buf_bytes),
+                           buf, dummy, wave, off);
+        }
+        // The records of the next iteration: they arrive under its wait.
+        ++jc;
+        const PageRec ncpl = jc + 1 < end ? pv_rec(p, jc + 1) : cur;
+        const PageRec nnxt = j + 2 < end ? pv_rec(p, j + 2) : cur;
+        const int par = (j - beg) & 1;
+        const uint32_t vbuf = buf + PV_V0 * 1024;  // the page's V granule columns
+        const uint4 pa = *(const uint4*)&s_p[par][0][lane][0];
+        const int jx = jb + 1 == p.nbuf ? 0 : jb + 1;  // the next page's buffer
+        if (j + 1 < end) form_p(nxt, base + (uint32_t)(jx * p.buf_bytes), 1 - par);
+        if constexpr (FMT == FMT_BF16) {
+            const bf16x8_t ahi = __builtin_bit_cast(bf16x8_t, pa);
+            const bf16x8_t alo = __builtin_bit_cast(bf16x8_t, *(const uint4*)&s_p[par][FMT == FMT_BF16 ? 1 : 0][lane][0]);
 #pragma unroll
             for (int i = 0; i < MB; ++i) {
                 const int cb = wave + NWAVE * i;
@@ -321,7 +332,7 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
                 }
             }
         } else if constexpr (FMT == FMT_F16) {
-            const half8_t av = to_f16x8(pe);
+            const half8_t av = __builtin_bit_cast(half8_t, pa);
 #pragma unroll
             for (int i = 0; i < MB; ++i) {
                 const int cb = wave + NWAVE * i;
@@ -333,7 +344,7 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
                 }
             }
         } else {
-            const half8_t av = to_f16x8(pe);
+            const half8_t av = __builtin_bit_cast(half8_t, pa);
             // This lane's 8 tokens' V scales as fp16 pairs (tokens 2j, 2j + 1), per kind.
             uint32_t so[4], si[4];
 #pragma unroll
@@ -408,10 +419,12 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
                 }
             }
         }
-        cur = ncur;
-        cpy = ncpy;
-        if (MULTI && seg_end && j + 1 < end) msk = sub_mask(pr_b(cur.bits));
-        jb = jb + 1 == p.nbuf ? 0 : jb + 1;
+        cur = nxt;
+        nxt = nnxt;
+        cpy = cpl;
+        cpl = ncpl;
+        if (MULTI && (cur.bits & PR_LAST) != 0 && j + 2 < end) msk = sub_mask(pr_b(nxt.bits));
+        jb = jx;
     }
     wait_vmcnt_lgkm0(0);  // no copy may land after the workgroup ends
 }
