@@ -127,7 +127,6 @@ __device__ __forceinline__ void pv_copies(const PvParams& p, const PvPage& d, ui
                                           int wave, const uint32_t (&off)[NLD]) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-        if (i >= p.nld) break;
         const int ch = i * NWAVE + wave;
         if (i == 0 && wave < PV_V0)
             lds_copy16(wave < 2 ? d.rl : d.rm, lbuf + (uint32_t)ch * 1024u, off[i]);
@@ -149,6 +148,18 @@ __device__ __forceinline__ uint2 tr_read8(uint32_t addr) {
 // as their high bytes, minus 1032 (all exact).
 __device__ __forceinline__ half2_t nib2(uint32_t w, uint32_t sel) {
     return as_h2(__builtin_amdgcn_perm(0x64646464u, w, sel)) - (half2_t){(_Float16)1032.f, (_Float16)1032.f};
+}
+
+// Waits for all but the copies of nbuf - 2 pages, NLD each; the usual counts without the table of
+// waits that a run-time count takes.
+template <int NLD>
+__device__ __forceinline__ void pv_wait(int nbuf) {
+    if (6 * NLD <= 63 && nbuf == 8)
+        SKV_WAIT_VM_LGKM0((6 * NLD) & 63);
+    else if (nbuf == 3)
+        SKV_WAIT_VM_LGKM0(NLD);
+    else
+        wait_vmcnt_lgkm0_wide((nbuf - 2) * NLD);
 }
 
 template <int FMT, int MB, int NLD, bool MULTI>
@@ -293,14 +304,14 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
             at[0] = __builtin_bit_cast(uint16_t, (_Float16)pe);
         }
     };
-    wait_vmcnt_lgkm0_wide((p.nbuf - 1) * p.nld);  // page beg's logits have landed
+    wait_vmcnt_lgkm0_wide((p.nbuf - 1) * NLD);  // page beg's logits have landed
     wait_lgkm0_barrier();
     form_p(cur, base, 0);
     if (MULTI && beg + 1 < end) msk = sub_mask(pr_b(nxt.bits));
     for (int j = beg; j < end; ++j) {
         // Page j's V is in buffer jb and page j + 1's logits in the next; the copies of the
         // nbuf - 2 pages after them may still run.
-        wait_vmcnt_lgkm0_wide((p.nbuf - 2) * p.nld);
+        pv_wait<NLD>(p.nbuf);
         wait_lgkm0_barrier();  // every wave is done with the previous page's buffer, P of page j is whole
         const uint32_t buf = base + (uint32_t)(jb * p.buf_bytes);
         {
@@ -807,17 +818,30 @@ constexpr int PV_NLD = 12;  // copies per wave per page, at most (the plan keeps
 // (115 KB) took 346 us.
 constexpr int PV_INFLIGHT = 64 * 1024;
 
+// Copies per wave and page: the smallest of 2, 4, 6 and 12 that holds them (a page loop with the
+// count known spends no scalar work on it: 64 x 8192, V rank 1290 3.2-bit 210 -> 192 us; copies
+// past the page's chunks read nothing).
+int pv_nld(int nld) { return nld <= 2 ? 2 : nld <= 4 ? 4 : nld <= 6 ? 6 : PV_NLD; }
+
+template <int FMT, bool MULTI, int NLD>
+const void* pv_pick_mb(int mb) {
+    if (mb <= 2) return (const void*)&pv_kernel<FMT, 2, NLD, MULTI>;
+    if (mb <= 4) return (const void*)&pv_kernel<FMT, 4, NLD, MULTI>;
+    if (mb <= 6) return (const void*)&pv_kernel<FMT, 6, NLD, MULTI>;
+    return (const void*)&pv_kernel<FMT, 8, NLD, MULTI>;
+}
+
 template <int FMT, bool MULTI>
-const void* pv_pick(int mb) {
-    if (mb <= 2) return (const void*)&pv_kernel<FMT, 2, PV_NLD, MULTI>;
-    if (mb <= 4) return (const void*)&pv_kernel<FMT, 4, PV_NLD, MULTI>;
-    if (mb <= 6) return (const void*)&pv_kernel<FMT, 6, PV_NLD, MULTI>;
-    return (const void*)&pv_kernel<FMT, 8, PV_NLD, MULTI>;
+const void* pv_pick(int mb, int nld) {
+    if (nld == 2) return pv_pick_mb<FMT, MULTI, 2>(mb);
+    if (nld == 4) return pv_pick_mb<FMT, MULTI, 4>(mb);
+    if (nld == 6) return pv_pick_mb<FMT, MULTI, 6>(mb);
+    return pv_pick_mb<FMT, MULTI, PV_NLD>(mb);
 }
 
 template <int FMT>
-const void* pv_pick_r(int mb, int r) {
-    return r > 1 ? pv_pick<FMT, true>(mb) : pv_pick<FMT, false>(mb);
+const void* pv_pick_r(int mb, int r, int nld) {
+    return r > 1 ? pv_pick<FMT, true>(mb, nld) : pv_pick<FMT, false>(mb, nld);
 }
 
 int raise_lds(const void* fn, int bytes) {
@@ -888,7 +912,7 @@ static PvPlan pv_plan(int fmt, int v_col, int v_rank, int vs_off, int vq_off, in
             pl.per = per;
             pl.nbuf = nbuf;
             pl.nch = nch;
-            pl.nld = (nch + NWAVE - 1) / NWAVE;
+            pl.nld = pv_nld((nch + NWAVE - 1) / NWAVE);
             pl.lds = nbuf * nch * 1024 + 1024;
             pl.ng = ng;
             pl.q_u1 = q_win ? 1 : 0;
@@ -928,9 +952,9 @@ int launch_pv(const DecodeParams& p, int fmt, int grid, hipStream_t stream) {
     a.v_off = pl.v_off;
     const int windows = (pl.units + pl.per - 1) / pl.per;
     const int mb = fmt == FMT_Q4 ? 2 * ((pl.per + NWAVE - 1) / NWAVE) : (pl.per + NWAVE - 1) / NWAVE;
-    const void* fn = fmt == FMT_BF16 ? pv_pick_r<FMT_BF16>(mb, p.pv_r)
-                     : fmt == FMT_F16 ? pv_pick_r<FMT_F16>(mb, p.pv_r)
-                                      : pv_pick_r<FMT_Q4>(mb, p.pv_r);
+    const void* fn = fmt == FMT_BF16 ? pv_pick_r<FMT_BF16>(mb, p.pv_r, pl.nld)
+                     : fmt == FMT_F16 ? pv_pick_r<FMT_F16>(mb, p.pv_r, pl.nld)
+                                      : pv_pick_r<FMT_Q4>(mb, p.pv_r, pl.nld);
     int rc = raise_lds(fn, PV_MAX_DYN_LDS);
     if (rc) return rc;
     void* args[] = {(void*)&a};
