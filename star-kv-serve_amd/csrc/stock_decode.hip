@@ -268,8 +268,9 @@ const void* stock_pick(int gw) {
 }
 
 // Splits per (request, head group): enough workgroups to fill the device (2 per CU), at
-// least 8 pages per split, at most ST_MAX_SPLITS. groups = workgroups per request and split.
-int stock_splits(int n, int groups, int max_seq_len) {
+// least 8 pages per split, at most ST_MAX_SPLITS. groups = workgroups per request and split;
+// mha: one query head per KV head.
+int stock_splits(int n, int groups, int max_seq_len, bool mha) {
     const int pages = (max_seq_len + 15) / 16;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -282,6 +283,17 @@ int stock_splits(int n, int groups, int max_seq_len) {
     // them, avoid a part-full last round (one request of 16384 tokens: 52.3 us, against
     // 57.4 us with the grid sized for three).
     int s = (int)std::min<int64_t>((2 * (int64_t)cus + wgs - 1) / wgs, (int64_t)(pages + 7) / 8);
+    // More than one workgroup a CU and long requests, one query head per KV head (the kernel that
+    // waits for memory): 3 splits, or 5 where the heads alone are less than a round, so that a round
+    // is less of the whole and a batch's longest requests are not one workgroup's work a head. Odd
+    // counts: workgroups are dealt to the XCDs by split first, and with an even count an XCD sees
+    // the same splits only, of which a short request's later ones are empty. One split against 3
+    // (5), us, equal lengths / ragged: 9 x 8192 305 / 210 against (239 / 171), 12 x 8192 354 / 274
+    // against (319 / 209), 16 x 8192 415 / 294 against 411 / 267, 20 x 8192 662 / 409 against 486 /
+    // 324, 24 x 3072 280 against 248, 64 x 4096 806 / 536 against 780 / 501. Whole rounds of short
+    // requests stay as they are: 16 x 3072 169 / 131 against 174 / 133, 64 x 2048 422 / 292 against
+    // 414 / 299.
+    if (mha && wgs > cus && pages >= 192 && (wgs % (2 * cus) != 0 || pages >= 256)) s = wgs < 2 * cus ? 5 : 3;
     s = std::min(s, ST_MAX_SPLITS);
     return s < 1 ? 1 : s;
 }
@@ -296,7 +308,8 @@ extern "C" {
 
 size_t starkv_stock_decode_workspace_bytes(int n, int num_heads, int num_kv_heads, int max_seq_len) {
     if (n < 1 || num_heads < 1 || num_kv_heads < 1 || max_seq_len < 1) return 0;
-    const int splits = stock_splits(n, num_heads == num_kv_heads ? num_heads : num_heads / 2, max_seq_len);
+    const int splits = stock_splits(n, num_heads == num_kv_heads ? num_heads : num_heads / 2, max_seq_len,
+                                    num_heads == num_kv_heads);
     return splits == 1 ? 256 : (size_t)n * num_heads * splits * 130 * 4;
 }
 
@@ -327,7 +340,7 @@ int starkv_stock_decode(void* stream, const void* query, int64_t q_s0, int64_t q
     SKV_CHECK(q_s0 % 8 == 0 && q_s1 % 8 == 0 && ((uintptr_t)query % 16) == 0,
               "stock_decode: query rows must be 16-byte aligned");
     const int gw = G == 1 ? 1 : 2;
-    const int splits = stock_splits(n, num_heads / gw, max_seq_len);
+    const int splits = stock_splits(n, num_heads / gw, max_seq_len, gw == 1);
     const size_t need = starkv_stock_decode_workspace_bytes(n, num_heads, num_kv_heads, max_seq_len);
     SKV_CHECK(workspace_bytes >= need, "stock_decode: workspace %zu bytes < %zu", workspace_bytes, need);
     StockParams p;

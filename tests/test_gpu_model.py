@@ -220,3 +220,30 @@ def test_stock_write_matches_index_put(cuda, slot_dtype):
     write_kv_full(k, v, kc, vc, slots)
     torch.cuda.synchronize()
     assert torch.equal(kc, want_k) and torch.equal(vc, want_v)
+
+
+@pytest.mark.parametrize("lens", [[3100, 1, 16, 2049, 0, 700, 3099, 17, 5], [3072 + 64 * i for i in range(17)]])
+def test_stock_decode_splits_of_larger_batches(cuda, lens):
+    """More (request, head) pairs than CUs with long spans: 5 splits (9 requests) and 3 (17), some of
+    them past a request's end, an empty request (NaN). Against float64 in torch, and by the decode
+    tolerance."""
+    g = torch.Generator().manual_seed(len(lens))
+    H, bs, n = 32, 16, len(lens)
+    pages = [(L + bs - 1) // bs for L in lens]
+    nb = sum(pages) + 1
+    kc, vc = (torch.randn(nb, bs, H, 128, generator=g).to(torch.bfloat16).to(cuda) for _ in range(2))
+    bt, o = torch.zeros(n, max(pages), dtype=torch.int32), 1
+    for b, p in enumerate(pages):
+        bt[b, :p] = torch.arange(o, o + p)
+        o += p
+    q = torch.randn(n, H, 128, generator=g).to(torch.bfloat16).to(cuda)
+    out = paged_decode_full(q, kc, vc, bt.to(cuda), torch.tensor(lens, dtype=torch.int32, device=cuda), max(lens),
+                            128 ** -0.5)
+    live = [b for b in range(n) if lens[b]]
+    truth = torch.empty(len(live), H, 128, dtype=torch.float64, device=cuda)
+    for i, b in enumerate(live):
+        K, V = (t[bt[b, :pages[b]].long().to(cuda)].reshape(-1, H, 128)[:lens[b]].double() for t in (kc, vc))
+        for h in range(H):
+            truth[i, h] = torch.softmax(K[:, h] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, h]
+    assert_close(out[live], truth.cpu().numpy(), f"stock splits n={n}")
+    assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
