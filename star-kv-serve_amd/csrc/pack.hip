@@ -134,8 +134,8 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const PackParams p) {
 // reductions inside the row, a lane packs every 16th byte), all lanes the V latent; the finished
 // row, assembled in LDS, goes out in whole 4-byte words. Against one wave per (token, head), whose
 // 64 lanes met heads of 16 to 48 codes and stored single bytes (32 heads, W 880, V rank 1290,
-// replayed from a graph): 4096 tokens 64.6 -> 22.3 us, 256 13.4 -> 6.1, one 10.2 -> 5.5. The
-// bound is the instructions of the quantizer (its divisions are exact).
+// replayed from a graph): 4096 tokens 64.6 -> 20.5 us, 256 13.4 -> 5.9, one 10.2 -> 5.4. The
+// bound is the instructions of the quantizer.
 // ---------------------------------------------------------------------------
 template <int DT>
 struct PackElem { typedef uint16_t T; };
@@ -207,8 +207,7 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const PackParams p) {
         for (int kb = l16; 2 * kb < wh; kb += 16) {
             const int l = 2 * kb;
             const float x0 = val(s_k[o + l]), x1 = val(s_k[o + l + 1]);
-            const int n0 = l < no ? quant_code(x0, s.s_out, -8.f, 7.f) : quant_code(x0, s.s_in, -4.f, 3.f);
-            const int n1 = l + 1 < no ? quant_code(x1, s.s_out, -8.f, 7.f) : quant_code(x1, s.s_in, -4.f, 3.f);
+            const int n0 = quant_code_of(x0, l < no, s), n1 = quant_code_of(x1, l + 1 < no, s);
             s_row[o / 2 + kb] = (uint8_t)(n0 | (n1 << 4));
         }
         if (l16 == 0) {

@@ -20,10 +20,23 @@ __device__ __forceinline__ int64_t load_slot(const void* slots, int bits, int i)
     return s < 0 ? 0 : s;
 }
 
+// clamp(rint(x / s)) + 8 with the division rounded once. |x| <= 7 s in a block, so the product with
+// the approximate reciprocal is within 2^-18 of the quotient: 2^-17 and more away from a midpoint
+// it rounds to the same integer, and only else (or for inf and NaN) is the division made.
 __device__ __forceinline__ int quant_code(float x, float s, float lo, float hi) {
-    float q = rintf(__fdiv_rn(x, s));
+    const float y = x * __builtin_amdgcn_rcpf(s);
+    float q = rintf(y);
+    if (!(fabsf(y - q) < 0.5f - 0x1p-17f)) q = rintf(__fdiv_rn(x, s));
     q = fminf(fmaxf(q, lo), hi);
     return (int)(q + 8.0f);
+}
+
+// Scales of a block's outliers and inliers.
+struct VScales {
+    float s_out, s_in;
+};
+__device__ __forceinline__ int quant_code_of(float x, bool outlier, const VScales& s) {
+    return quant_code(x, outlier ? s.s_out : s.s_in, outlier ? -8.f : -4.f, outlier ? 7.f : 3.f);
 }
 
 // K block of KV head u: rank R, `nout` outlier lanes, first lane `off` of the row;
@@ -45,8 +58,8 @@ __device__ __forceinline__ void pack_k_block(Src&& src, int R, int nout, int off
     const float s_in = __fdiv_rn(a_in, 3.0f);
     for (int kb = lane; 2 * kb < wh; kb += 64) {
         const int l = 2 * kb;
-        const int n0 = l < nout ? quant_code(src(l), s_out, -8.f, 7.f) : quant_code(src(l), s_in, -4.f, 3.f);
-        const int n1 = l + 1 < nout ? quant_code(src(l + 1), s_out, -8.f, 7.f) : quant_code(src(l + 1), s_in, -4.f, 3.f);
+        const VScales s{s_out, s_in};
+        const int n0 = quant_code_of(src(l), l < nout, s), n1 = quant_code_of(src(l + 1), l + 1 < nout, s);
         row[off / 2 + kb] = (uint8_t)(n0 | (n1 << 4));
     }
     if (lane == 0) {
@@ -61,9 +74,6 @@ __device__ __forceinline__ void pack_k_block(Src&& src, int R, int nout, int off
 // [vq_off + nb, row_bytes) are written as zero (the reference leaves them unwritten).
 // The pieces (scales from the two maxima, one byte, the tail) are shared with the
 // direct write, which packs a row's bytes over several workgroups.
-struct VScales {
-    float s_out, s_in;
-};
 // a_out / a_in: max |x| over the outlier / inlier channels (0 when there are none).
 __device__ __forceinline__ VScales v_scales(float a_out, float a_in) {
     return VScales{__fdiv_rn(fmaxf(a_out, 1e-5f), 7.0f), __fdiv_rn(fmaxf(a_in, 1e-5f), 3.0f)};

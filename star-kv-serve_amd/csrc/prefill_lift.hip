@@ -17,7 +17,8 @@
 // the bound is that and the latency of a wave's few dependent loads.
 // At 32 heads and W = 880, traced: 4096 tokens 31 us where those launches (a gather, conversions, a
 // transposed copy, the product, six elementwise kernels, a concatenation) took 233; 6368 tokens in
-// 7 prompts 39 us against 366.
+// 7 prompts 39 us against 366. With the cos/sin values read after the products (96 registers, five
+// waves a SIMD instead of two) 26 and 36 us.
 // The V planes (grid.y past the head groups) convert the V codes of 32 tokens.
 #include "decode_pages.hpp"
 
@@ -137,7 +138,7 @@ __device__ __forceinline__ float2 lift_rotate(float x1, float x2, float c, float
 }
 
 template <int DT, int CDT>
-__global__ __launch_bounds__(64 * LIFT_WAVES) void prefill_lift_kernel(const LiftParams p) {
+__global__ __launch_bounds__(64 * LIFT_WAVES, CDT == STARKV_F32 ? 3 : 4) void prefill_lift_kernel(const LiftParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t s_rows[LIFT_WAVES][LIFT_TOK * 256];
     const int lane = threadIdx.x & 63, wave = rfl(threadIdx.x >> 6);
     const int t0 = blockIdx.x * LIFT_TOK;
@@ -161,13 +162,6 @@ __global__ __launch_bounds__(64 * LIFT_WAVES) void prefill_lift_kernel(const Lif
         if (p.cu[mid] <= t) lo = mid; else hi = mid - 1;
     }
     const int64_t row = (int64_t)(t - p.cu[lo]) * p.cs_s0 + 16 * hh;
-    LiftTrig<CDT> cs[2], sn[2];  // dimensions 32 j + 16 hh .. + 15
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        cs[j].load(p.cs, row + 32 * j);
-        sn[j].load(p.cs, row + 64 + 32 * j);
-    }
-
     const int64_t code = (int64_t)t * p.k_s0 + off;
     const float* u = p.u + (int64_t)off * p.u_s0 + 4 * n;
     f32x16_t z[4];
@@ -176,17 +170,27 @@ __global__ __launch_bounds__(64 * LIFT_WAVES) void prefill_lift_kernel(const Lif
 #pragma unroll 1
     for (int r0 = 0; r0 < width; r0 += 16) {
         float x[8];
-        float4 a[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) a[s] = *(const float4*)(u + (int64_t)min(r0 + lift_rank(s, hh), width - 1) * p.u_s0);
         lift_codes<DT>(p.k, code, r0, width, hh, x);
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            z[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].x, x[s], z[0], 0, 0, 0);
-            z[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].y, x[s], z[1], 0, 0, 0);
-            z[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].z, x[s], z[2], 0, 0, 0);
-            z[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].w, x[s], z[3], 0, 0, 0);
+        for (int g = 0; g < 2; ++g) {
+            float4 a[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                a[s] = *(const float4*)(u + (int64_t)min(r0 + lift_rank(4 * g + s, hh), width - 1) * p.u_s0);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                z[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].x, x[4 * g + s], z[0], 0, 0, 0);
+                z[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].y, x[4 * g + s], z[1], 0, 0, 0);
+                z[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].z, x[4 * g + s], z[2], 0, 0, 0);
+                z[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s].w, x[4 * g + s], z[3], 0, 0, 0);
+            }
         }
+    }
+    LiftTrig<CDT> cs[2], sn[2];  // dimensions 32 j + 16 hh .. + 15
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        cs[j].load(p.cs, row + 32 * j);
+        sn[j].load(p.cs, row + 64 + 32 * j);
     }
     // z[b][4 j + e] is dimension 32 j + 16 hh + 4 e + b of token n; j + 2 holds the partners.
     uint8_t* rows = s_rows[wave];
