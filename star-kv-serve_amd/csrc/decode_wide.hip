@@ -48,7 +48,7 @@ namespace starkv {
 
 namespace {
 
-constexpr int PV_MAX_DYN_LDS = 160 * 1024 - 4096;  // beside at most 4 KB of P
+constexpr int PV_MAX_DYN_LDS = 160 * 1024 - 8192;  // beside at most 8 KB of P
 
 // Swizzled slot of token t in granule column G.
 __device__ __forceinline__ int gslot(int G, int t) { return t ^ ((G & 1) << 2); }
@@ -150,24 +150,26 @@ __device__ __forceinline__ half2_t nib2(uint32_t w, uint32_t sel) {
     return as_h2(__builtin_amdgcn_perm(0x64646464u, w, sel)) - (half2_t){(_Float16)1032.f, (_Float16)1032.f};
 }
 
-// Waits for all but the copies of nbuf - 2 pages, NLD each; the usual counts without the table of
-// waits that a run-time count takes.
-template <int NLD>
+// Waits for all but the copies of nbuf - 2 PG pages, NLD each; the usual counts without the table
+// of waits that a run-time count takes.
+template <int NLD, int PG>
 __device__ __forceinline__ void pv_wait(int nbuf) {
-    if (6 * NLD <= 63 && nbuf == 8)
-        SKV_WAIT_VM_LGKM0((6 * NLD) & 63);
-    else if (nbuf == 3)
-        SKV_WAIT_VM_LGKM0(NLD);
+    constexpr int A = PG == 2 ? 8 : 3, B = PG == 2 ? 6 : 4;  // the usual numbers of buffers
+    if (nbuf == A)
+        SKV_WAIT_VM_LGKM0((A - 2 * PG) * NLD);
+    else if (nbuf == B)
+        SKV_WAIT_VM_LGKM0((B - 2 * PG) * NLD);
     else
-        wait_vmcnt_lgkm0_wide((nbuf - 2) * NLD);
+        wait_vmcnt_lgkm0_wide((nbuf - 2 * PG) * NLD);
 }
 
-template <int FMT, int MB, int NLD, bool MULTI>
+// PG: pages between barriers (2 where at least 6 buffers fit).
+template <int FMT, int MB, int NLD, bool MULTI, int PG>
 __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_pv[];
-    // P of the current and the next page as the MFMA's A operand: [page parity][bf16: high and
-    // low parts][lane][8].
-    __shared__ __attribute__((aligned(16))) uint16_t s_p[2][FMT == FMT_BF16 ? 2 : 1][64][8];
+    // P of the current and the next PG pages as the MFMA's A operand: [page][bf16: high and low
+    // parts][lane][8].
+    __shared__ __attribute__((aligned(16))) uint16_t s_p[2 * PG][FMT == FMT_BF16 ? 2 : 1][64][8];
     // The parameters by value: the page loop's fields stay in registers (this kernel has
     // the registers to spare) instead of being reloaded where they are used.
     const PvParams& p = p0;
@@ -243,27 +245,35 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[i] = (f32x16_t){};
 
-    // Records: the current page j (cur) and the next (nxt); the page whose V copies issue in
-    // iteration j (cpy = page j + nbuf - 1) and the one after it, whose logits do (cpl). Each is
-    // loaded an iteration before its use.
-    PageRec cur = pv_rec(p, beg), nxt = beg + 1 < end ? pv_rec(p, beg + 1) : cur;
-    // Prologue: the logits of page beg, then V of pages beg .. beg + nbuf - 2, each with the next
-    // page's logits, in flight.
+    // Records: the current pages j + u (cur), u < PG, and the next PG (nxt); the pages whose V
+    // copies issue in this iteration (cpy = pages j + nbuf - PG + u) and the PG after them, whose
+    // logits do (cpl). Each is loaded an iteration before its use.
+    auto rec_at = [&](int j) { return pv_rec(p, j < end ? j : beg); };
+    PageRec cur[PG], nxt[PG], cpy[PG], cpl[PG];
+    int jc = beg + p.nbuf - PG;  // the first page whose V copies issue next
+#pragma unroll
+    for (int u = 0; u < PG; ++u) {
+        cur[u] = rec_at(beg + u);
+        nxt[u] = rec_at(beg + PG + u);
+    }
+    // Prologue: the logits of the first PG pages, then V of pages beg .. beg + nbuf - PG - 1, each
+    // with the logits of the page PG further on, in flight.
     if (wave < PV_V0) {
-        const PvPage d = pv_page_desc(p, cur, false, cur, true, g);
-        lds_copy16(wave < 2 ? d.rl : d.rm, base + (uint32_t)wave * 1024u, off[0]);
+#pragma unroll
+        for (int u = 0; u < PG; ++u) {
+            const PvPage d = pv_page_desc(p, cur[u], false, cur[u], beg + u < end, g);
+            lds_copy16(wave < 2 ? d.rl : d.rm, base + (uint32_t)(u * p.buf_bytes + wave * 1024), off[0]);
+        }
     }
-    PageRec cpy = cur;
-    for (int j = 0; j < p.nbuf - 1; ++j) {
-        const bool v = beg + j < end, vn = beg + j + 1 < end;
-        const PageRec rn = vn ? pv_rec(p, beg + j + 1) : cur;
-        pv_copies<NLD>(p, pv_page_desc(p, cpy, v, rn, vn, g), base + (uint32_t)(j * p.buf_bytes),
-                       base + (uint32_t)((j + 1) * p.buf_bytes), dummy, wave, off);
-        cpy = rn;
+    for (int j = 0; j < p.nbuf - PG; ++j)
+        pv_copies<NLD>(p, pv_page_desc(p, rec_at(beg + j), beg + j < end, rec_at(beg + j + PG), beg + j + PG < end, g),
+                       base + (uint32_t)(j * p.buf_bytes), base + (uint32_t)((j + PG) * p.buf_bytes), dummy, wave, off);
+#pragma unroll
+    for (int u = 0; u < PG; ++u) {
+        cpy[u] = rec_at(jc + u);
+        cpl[u] = rec_at(jc + PG + u);
     }
-    int jc = beg + p.nbuf - 1;  // the page whose V copies issue next
-    PageRec cpl = jc + 1 < end ? pv_rec(p, jc + 1) : cur;
-    int jb = 0;  // buffer of the current page
+    int jb = 0;  // buffer of page j
     // The logits-pass ranges R g + j holding pages of request b: bit j. This pass's
     // reference max of the request is the largest of theirs (slots of other ranges hold
     // other requests' values, or none).
@@ -277,9 +287,13 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
         }
         return msk;
     };
-    int msk = sub_mask(pr_b(cur.bits));  // of the next page's request, redone when the request changes
-    // P of a page (its record r, its logits in the buffer at lbuf) into s_p[par]: one value a lane.
-    auto form_p = [&](const PageRec& r, uint32_t lbuf, int par) {
+    int msk = 1, msk_b = -1;  // of request msk_b
+    // P of a page (its record r, its logits in the buffer at lbuf) into s_p[to]: one value a lane.
+    auto form_p = [&](const PageRec& r, uint32_t lbuf, int to) {
+        if (MULTI && pr_b(r.bits) != msk_b) {
+            msk_b = pr_b(r.bits);
+            msk = sub_mask(msk_b);
+        }
         // R = 1: the slot's max. Else the largest of the R slots' maxima (all four read:
         // the slots past R are in the chunk too), those of other requests' ranges left out.
         float mx;
@@ -295,7 +309,7 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
         }
         const bool ok = ph < p.Hq && pt < pr_rows(r.bits);
         const float pe = __builtin_amdgcn_exp2f(ok ? lds_ld<float>(lbuf + lga) - mx : -INFINITY);  // exp2(-inf) = 0
-        uint16_t* at = pput + par * (int)(sizeof(s_p[0]) / 2);
+        uint16_t* at = pput + to * (int)(sizeof(s_p[0]) / 2);
         if constexpr (FMT == FMT_BF16) {
             const __bf16 hi = (__bf16)pe;
             at[0] = __builtin_bit_cast(uint16_t, hi);
@@ -304,137 +318,155 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
             at[0] = __builtin_bit_cast(uint16_t, (_Float16)pe);
         }
     };
-    wait_vmcnt_lgkm0_wide((p.nbuf - 1) * NLD);  // page beg's logits have landed
+    wait_vmcnt_lgkm0_wide((p.nbuf - PG) * NLD);  // the first pages' logits have landed
     wait_lgkm0_barrier();
-    form_p(cur, base, 0);
-    if (MULTI && beg + 1 < end) msk = sub_mask(pr_b(nxt.bits));
-    for (int j = beg; j < end; ++j) {
-        // Page j's V is in buffer jb and page j + 1's logits in the next; the copies of the
-        // nbuf - 2 pages after them may still run.
-        pv_wait<NLD>(p.nbuf);
-        wait_lgkm0_barrier();  // every wave is done with the previous page's buffer, P of page j is whole
+#pragma unroll
+    for (int u = 0; u < PG; ++u)
+        if (beg + u < end) form_p(cur[u], base + (uint32_t)(u * p.buf_bytes), u);
+    int par = 0;
+    for (int j = beg; j < end; j += PG) {
+        // V of pages j + u is in buffers jb + u and the next PG pages' logits in the buffers after
+        // them; the copies of the nbuf - 2 PG pages after those may still run.
+        pv_wait<NLD, PG>(p.nbuf);
+        wait_lgkm0_barrier();  // every wave is done with the previous pages' buffers, P of these is whole
         const uint32_t buf = base + (uint32_t)(jb * p.buf_bytes);
-        {
-            const int jn = jb == 0 ? p.nbuf - 1 : jb - 1;  // the buffer whose V the previous page used
-            pv_copies<NLD>(p, pv_page_desc(p, cpy, jc < end, cpl, jc + 1 < end, g), base + (uint32_t)(jn * p.buf_bytes),
-                           buf, dummy, wave, off);
-        }
+        const uint32_t bprev = base + (uint32_t)((jb == 0 ? p.nbuf - PG : jb - PG) * p.buf_bytes);
+#pragma unroll
+        for (int u = 0; u < PG; ++u)
+            pv_copies<NLD>(p, pv_page_desc(p, cpy[u], jc + u < end, cpl[u], jc + PG + u < end, g),
+                           bprev + (uint32_t)(u * p.buf_bytes), buf + (uint32_t)(u * p.buf_bytes), dummy, wave, off);
         // The records of the next iteration: they arrive under its wait.
-        ++jc;
-        const PageRec ncpl = jc + 1 < end ? pv_rec(p, jc + 1) : cur;
-        const PageRec nnxt = j + 2 < end ? pv_rec(p, j + 2) : cur;
-        const int par = (j - beg) & 1;
-        const uint32_t vbuf = buf + PV_V0 * 1024;  // the page's V granule columns
-        const uint4 pa = *(const uint4*)&s_p[par][0][lane][0];
-        const int jx = jb + 1 == p.nbuf ? 0 : jb + 1;  // the next page's buffer
-        if (j + 1 < end) form_p(nxt, base + (uint32_t)(jx * p.buf_bytes), 1 - par);
-        if constexpr (FMT == FMT_BF16) {
-            const bf16x8_t ahi = __builtin_bit_cast(bf16x8_t, pa);
-            const bf16x8_t alo = __builtin_bit_cast(bf16x8_t, *(const uint4*)&s_p[par][FMT == FMT_BF16 ? 1 : 0][lane][0]);
+        jc += PG;
+        PageRec ncpl[PG], nnxt[PG];
 #pragma unroll
-            for (int i = 0; i < MB; ++i) {
-                const int cb = wave + NWAVE * i;
-                if (cb < ncb) {
-                    const uint32_t a = vbuf + (uint32_t)cb * 1024u;
-                    const uint2 b0 = tr_read(a + trd0), b1 = tr_read(a + trd1);
-                    const bf16x8_t bv = __builtin_bit_cast(bf16x8_t, make_uint4(b0.x, b0.y, b1.x, b1.y));
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bv, acc[i], 0, 0, 0);
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo, bv, acc[i], 0, 0, 0);
-                }
-            }
-        } else if constexpr (FMT == FMT_F16) {
-            const half8_t av = __builtin_bit_cast(half8_t, pa);
-#pragma unroll
-            for (int i = 0; i < MB; ++i) {
-                const int cb = wave + NWAVE * i;
-                if (cb < ncb) {
-                    const uint32_t a = vbuf + (uint32_t)cb * 1024u;
-                    const uint2 b0 = tr_read(a + trd0), b1 = tr_read(a + trd1);
-                    const half8_t bv = __builtin_bit_cast(half8_t, make_uint4(b0.x, b0.y, b1.x, b1.y));
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc[i], 0, 0, 0);
-                }
-            }
-        } else {
-            const half8_t av = __builtin_bit_cast(half8_t, pa);
-            // This lane's 8 tokens' V scales as fp16 pairs (tokens 2j, 2j + 1), per kind.
-            uint32_t so[4], si[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = 8 * ag + 2 * j;
-                const uint32_t w0 = lds_ld<uint32_t>(vbuf + (uint32_t)(gslot(0, t) * 16 + p.vs_rel));
-                const uint32_t w1 = lds_ld<uint32_t>(vbuf + (uint32_t)(gslot(0, t + 1) * 16 + p.vs_rel));
-                so[j] = h2_bits(cvt_h2(__uint_as_float(w0 << 16), __uint_as_float(w1 << 16)));
-                si[j] = h2_bits(cvt_h2(__uint_as_float(w0 & 0xffff0000u), __uint_as_float(w1 & 0xffff0000u)));
-            }
-            // Every chunk's bytes first (chunks past the window reread the last one, unused).
-            uint2 wv[MB / 2];
-#pragma unroll
-            for (int i = 0; i < MB / 2; ++i)
-                wv[i] = tr_read8(vbuf + (uint32_t)((p.q_u1 ? 1 : c0) + min(wave + NWAVE * i, ncb - 1)) * 512u + trd0);
-#pragma unroll
-            for (int i = 0; i < MB / 2; ++i) {
-                const int ch = wave + NWAVE * i;  // 32-byte chunk of the copied V bytes
-                if (ch < ncb) {
-                    const int c = c0 + ch;
-                    const uint2 w = wv[i];
-                    // This lane's byte: outlier columns before v_nbo bytes of nibbles, inlier after.
-                    const bool inl = 32 * c + (lane & 31) - p.vq_rel >= p.v_nbo;
-                    const uint32_t l0 = w.x & 0x0F0F0F0Fu, l1 = w.y & 0x0F0F0F0Fu;
-                    const uint32_t h0 = (w.x >> 4) & 0x0F0F0F0Fu, h1 = (w.y >> 4) & 0x0F0F0F0Fu;
-                    half2_t sc[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) sc[j] = as_h2(inl ? si[j] : so[j]);
-                    const half2_t e0 = nib2(l0, 0x04010400u) * sc[0], e1 = nib2(l0, 0x04030402u) * sc[1];
-                    const half2_t e2 = nib2(l1, 0x04010400u) * sc[2], e3 = nib2(l1, 0x04030402u) * sc[3];
-                    const half2_t o0 = nib2(h0, 0x04010400u) * sc[0], o1 = nib2(h0, 0x04030402u) * sc[1];
-                    const half2_t o2 = nib2(h1, 0x04010400u) * sc[2], o3 = nib2(h1, 0x04030402u) * sc[3];
-                    const half8_t be = __builtin_bit_cast(
-                        half8_t, make_uint4(h2_bits(e0), h2_bits(e1), h2_bits(e2), h2_bits(e3)));
-                    const half8_t bo = __builtin_bit_cast(
-                        half8_t, make_uint4(h2_bits(o0), h2_bits(o1), h2_bits(o2), h2_bits(o3)));
-                    acc[2 * i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, be, acc[2 * i], 0, 0, 0);
-                    acc[2 * i + 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bo, acc[2 * i + 1], 0, 0, 0);
-                }
-            }
+        for (int u = 0; u < PG; ++u) {
+            ncpl[u] = rec_at(jc + PG + u);
+            nnxt[u] = rec_at(j + 2 * PG + u);
         }
-        const bool seg_end = (cur.bits & PR_LAST) != 0 || j + 1 == end;
-        if (seg_end) {
-            // This lane's column of each of its blocks, for the 16 heads
-            // 8 (j / 4) + 4 (lane >> 5) + j % 4 of the 32x32 result.
-            const int64_t slot = (int64_t)pr_b(cur.bits) + g;
-            float* wa = (float*)(p.ws + p.ws_acc) + slot * p.Hq * p.acc_ld;
+        uint4 pa[PG], pl[PG];
 #pragma unroll
-            for (int i = 0; i < MB; ++i) {
-                int col = -1;
-                if (FMT == FMT_Q4) {
-                    const int ch = wave + NWAVE * (i >> 1);
-                    const int rel = 32 * (c0 + ch) + (lane & 31) - p.vq_rel;  // nibble byte of this lane
-                    if (ch < ncb && rel >= 0) {
-                        if (rel < p.v_nbo) {
-                            col = 2 * rel + (i & 1);
-                            if (col >= p.v_nout) col = -1;
-                        } else {
-                            col = p.v_nout + 2 * (rel - p.v_nbo) + (i & 1);
-                        }
-                    }
-                } else {
+        for (int u = 0; u < PG; ++u) {
+            pa[u] = *(const uint4*)&s_p[par * PG + u][0][lane][0];
+            if (FMT == FMT_BF16) pl[u] = *(const uint4*)&s_p[par * PG + u][FMT == FMT_BF16 ? 1 : 0][lane][0];
+        }
+        const int jx = jb + PG == p.nbuf ? 0 : jb + PG;  // the next pages' buffers
+#pragma unroll
+        for (int u = 0; u < PG; ++u)
+            if (j + PG + u < end) form_p(nxt[u], base + (uint32_t)((jx + u) * p.buf_bytes), (1 - par) * PG + u);
+#pragma unroll
+        for (int u = 0; u < PG; ++u) {
+            if (u > 0 && j + u >= end) break;
+            const uint32_t vbuf = buf + (uint32_t)(u * p.buf_bytes) + PV_V0 * 1024;  // the page's V granule columns
+            if constexpr (FMT == FMT_BF16) {
+                const bf16x8_t ahi = __builtin_bit_cast(bf16x8_t, pa[u]), alo = __builtin_bit_cast(bf16x8_t, pl[u]);
+#pragma unroll
+                for (int i = 0; i < MB; ++i) {
                     const int cb = wave + NWAVE * i;
-                    if (cb < ncb) col = c0 + 32 * cb + (lane & 31);
+                    if (cb < ncb) {
+                        const uint32_t a = vbuf + (uint32_t)cb * 1024u;
+                        const uint2 b0 = tr_read(a + trd0), b1 = tr_read(a + trd1);
+                        const bf16x8_t bv = __builtin_bit_cast(bf16x8_t, make_uint4(b0.x, b0.y, b1.x, b1.y));
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi, bv, acc[i], 0, 0, 0);
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo, bv, acc[i], 0, 0, 0);
+                    }
                 }
-                const bool okc = col >= 0 && col < p.v_rank;
+            } else if constexpr (FMT == FMT_F16) {
+                const half8_t av = __builtin_bit_cast(half8_t, pa[u]);
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int h = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-                    if (okc && h < p.Hq) wa[(int64_t)h * p.acc_ld + col] = acc[i][j];
-                    acc[i][j] = 0.f;
+                for (int i = 0; i < MB; ++i) {
+                    const int cb = wave + NWAVE * i;
+                    if (cb < ncb) {
+                        const uint32_t a = vbuf + (uint32_t)cb * 1024u;
+                        const uint2 b0 = tr_read(a + trd0), b1 = tr_read(a + trd1);
+                        const half8_t bv = __builtin_bit_cast(half8_t, make_uint4(b0.x, b0.y, b1.x, b1.y));
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc[i], 0, 0, 0);
+                    }
+                }
+            } else {
+                const half8_t av = __builtin_bit_cast(half8_t, pa[u]);
+                // This lane's 8 tokens' V scales as fp16 pairs (tokens 2j, 2j + 1), per kind.
+                uint32_t so[4], si[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int t = 8 * ag + 2 * j;
+                    const uint32_t w0 = lds_ld<uint32_t>(vbuf + (uint32_t)(gslot(0, t) * 16 + p.vs_rel));
+                    const uint32_t w1 = lds_ld<uint32_t>(vbuf + (uint32_t)(gslot(0, t + 1) * 16 + p.vs_rel));
+                    so[j] = h2_bits(cvt_h2(__uint_as_float(w0 << 16), __uint_as_float(w1 << 16)));
+                    si[j] = h2_bits(cvt_h2(__uint_as_float(w0 & 0xffff0000u), __uint_as_float(w1 & 0xffff0000u)));
+                }
+                // Every chunk's bytes first (chunks past the window reread the last one, unused).
+                uint2 wv[MB / 2];
+#pragma unroll
+                for (int i = 0; i < MB / 2; ++i)
+                    wv[i] = tr_read8(vbuf + (uint32_t)((p.q_u1 ? 1 : c0) + min(wave + NWAVE * i, ncb - 1)) * 512u + trd0);
+#pragma unroll
+                for (int i = 0; i < MB / 2; ++i) {
+                    const int ch = wave + NWAVE * i;  // 32-byte chunk of the copied V bytes
+                    if (ch < ncb) {
+                        const int c = c0 + ch;
+                        const uint2 w = wv[i];
+                        // This lane's byte: outlier columns before v_nbo bytes of nibbles, inlier after.
+                        const bool inl = 32 * c + (lane & 31) - p.vq_rel >= p.v_nbo;
+                        const uint32_t l0 = w.x & 0x0F0F0F0Fu, l1 = w.y & 0x0F0F0F0Fu;
+                        const uint32_t h0 = (w.x >> 4) & 0x0F0F0F0Fu, h1 = (w.y >> 4) & 0x0F0F0F0Fu;
+                        half2_t sc[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sc[j] = as_h2(inl ? si[j] : so[j]);
+                        const half2_t e0 = nib2(l0, 0x04010400u) * sc[0], e1 = nib2(l0, 0x04030402u) * sc[1];
+                        const half2_t e2 = nib2(l1, 0x04010400u) * sc[2], e3 = nib2(l1, 0x04030402u) * sc[3];
+                        const half2_t o0 = nib2(h0, 0x04010400u) * sc[0], o1 = nib2(h0, 0x04030402u) * sc[1];
+                        const half2_t o2 = nib2(h1, 0x04010400u) * sc[2], o3 = nib2(h1, 0x04030402u) * sc[3];
+                        const half8_t be = __builtin_bit_cast(
+                            half8_t, make_uint4(h2_bits(e0), h2_bits(e1), h2_bits(e2), h2_bits(e3)));
+                        const half8_t bo = __builtin_bit_cast(
+                            half8_t, make_uint4(h2_bits(o0), h2_bits(o1), h2_bits(o2), h2_bits(o3)));
+                        acc[2 * i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, be, acc[2 * i], 0, 0, 0);
+                        acc[2 * i + 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bo, acc[2 * i + 1], 0, 0, 0);
+                    }
+                }
+            }
+            const bool seg_end = (cur[u].bits & PR_LAST) != 0 || j + u + 1 == end;
+            if (seg_end) {
+                // This lane's column of each of its blocks, for the 16 heads
+                // 8 (j / 4) + 4 (lane >> 5) + j % 4 of the 32x32 result.
+                const int64_t slot = (int64_t)pr_b(cur[u].bits) + g;
+                float* wa = (float*)(p.ws + p.ws_acc) + slot * p.Hq * p.acc_ld;
+#pragma unroll
+                for (int i = 0; i < MB; ++i) {
+                    int col = -1;
+                    if (FMT == FMT_Q4) {
+                        const int ch = wave + NWAVE * (i >> 1);
+                        const int rel = 32 * (c0 + ch) + (lane & 31) - p.vq_rel;  // nibble byte of this lane
+                        if (ch < ncb && rel >= 0) {
+                            if (rel < p.v_nbo) {
+                                col = 2 * rel + (i & 1);
+                                if (col >= p.v_nout) col = -1;
+                            } else {
+                                col = p.v_nout + 2 * (rel - p.v_nbo) + (i & 1);
+                            }
+                        }
+                    } else {
+                        const int cb = wave + NWAVE * i;
+                        if (cb < ncb) col = c0 + 32 * cb + (lane & 31);
+                    }
+                    const bool okc = col >= 0 && col < p.v_rank;
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) {
+                        const int h = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+                        if (okc && h < p.Hq) wa[(int64_t)h * p.acc_ld + col] = acc[i][j];
+                        acc[i][j] = 0.f;
+                    }
                 }
             }
         }
-        cur = nxt;
-        nxt = nnxt;
-        cpy = cpl;
-        cpl = ncpl;
-        if (MULTI && (cur.bits & PR_LAST) != 0 && j + 2 < end) msk = sub_mask(pr_b(nxt.bits));
+#pragma unroll
+        for (int u = 0; u < PG; ++u) {
+            cur[u] = nxt[u];
+            nxt[u] = nnxt[u];
+            cpy[u] = cpl[u];
+            cpl[u] = ncpl[u];
+        }
+        par = 1 - par;
         jb = jx;
     }
     wait_vmcnt_lgkm0(0);  // no copy may land after the workgroup ends
@@ -822,26 +854,31 @@ constexpr int PV_INFLIGHT = 64 * 1024;
 // count known spends no scalar work on it: 64 x 8192, V rank 1290 3.2-bit 210 -> 192 us; copies
 // past the page's chunks read nothing).
 int pv_nld(int nld) { return nld <= 2 ? 2 : nld <= 4 ? 4 : nld <= 6 ? 6 : PV_NLD; }
+// Pages between barriers: with 6 buffers or more two keep four further pages in flight, and a
+// barrier, its wait and the loop's scalar work come once for both: 64 x 8192, V rank 1290 3.2-bit 192 ->
+// 187 us, one request of 16384 tokens 21.5 -> 20.3.
+int pv_pages(int nbuf) { return nbuf >= 6 ? 2 : 1; }
 
-template <int FMT, bool MULTI, int NLD>
+template <int FMT, bool MULTI, int NLD, int PG>
 const void* pv_pick_mb(int mb) {
-    if (mb <= 2) return (const void*)&pv_kernel<FMT, 2, NLD, MULTI>;
-    if (mb <= 4) return (const void*)&pv_kernel<FMT, 4, NLD, MULTI>;
-    if (mb <= 6) return (const void*)&pv_kernel<FMT, 6, NLD, MULTI>;
-    return (const void*)&pv_kernel<FMT, 8, NLD, MULTI>;
+    if (mb <= 2) return (const void*)&pv_kernel<FMT, 2, NLD, MULTI, PG>;
+    if (mb <= 4) return (const void*)&pv_kernel<FMT, 4, NLD, MULTI, PG>;
+    if (mb <= 6) return (const void*)&pv_kernel<FMT, 6, NLD, MULTI, PG>;
+    return (const void*)&pv_kernel<FMT, 8, NLD, MULTI, PG>;
 }
 
+// Six buffers hold pages of at most 25 chunks, 4 copies a wave; fewer buffers mean more than 3.
 template <int FMT, bool MULTI>
-const void* pv_pick(int mb, int nld) {
-    if (nld == 2) return pv_pick_mb<FMT, MULTI, 2>(mb);
-    if (nld == 4) return pv_pick_mb<FMT, MULTI, 4>(mb);
-    if (nld == 6) return pv_pick_mb<FMT, MULTI, 6>(mb);
-    return pv_pick_mb<FMT, MULTI, PV_NLD>(mb);
+const void* pv_pick(int mb, int nld, int pg) {
+    if (pg == 2) return nld == 2 ? pv_pick_mb<FMT, MULTI, 2, 2>(mb) : pv_pick_mb<FMT, MULTI, 4, 2>(mb);
+    if (nld <= 4) return pv_pick_mb<FMT, MULTI, 4, 1>(mb);
+    if (nld == 6) return pv_pick_mb<FMT, MULTI, 6, 1>(mb);
+    return pv_pick_mb<FMT, MULTI, PV_NLD, 1>(mb);
 }
 
 template <int FMT>
-const void* pv_pick_r(int mb, int r, int nld) {
-    return r > 1 ? pv_pick<FMT, true>(mb, nld) : pv_pick<FMT, false>(mb, nld);
+const void* pv_pick_r(int mb, int r, int nld, int pg) {
+    return r > 1 ? pv_pick<FMT, true>(mb, nld, pg) : pv_pick<FMT, false>(mb, nld, pg);
 }
 
 int raise_lds(const void* fn, int bytes) {
@@ -903,8 +940,9 @@ static PvPlan pv_plan(int fmt, int v_col, int v_rank, int vs_off, int vq_off, in
         const int ng = fmt == FMT_Q4 ? (q_win ? 2 + 2 * per : pl.ng_all) : 4 * per;
         const int nch = (ng + 3) / 4 + PV_V0;
         if ((nch + NWAVE - 1) / NWAVE > PV_NLD) continue;
-        const int nbuf = std::min(8, (PV_MAX_DYN_LDS - 1024) / (nch * 1024));
+        int nbuf = std::min(8, (PV_MAX_DYN_LDS - 1024) / (nch * 1024));
         if (nbuf < 2) continue;
+        nbuf -= nbuf % pv_pages(nbuf);
         const int inflight = (nbuf - 1) * nch * 1024;
         const int score = inflight >= PV_INFLIGHT && nbuf >= 3 ? (1 << 30) - launches : inflight;
         if (score > best_score) {
@@ -952,9 +990,11 @@ int launch_pv(const DecodeParams& p, int fmt, int grid, hipStream_t stream) {
     a.v_off = pl.v_off;
     const int windows = (pl.units + pl.per - 1) / pl.per;
     const int mb = fmt == FMT_Q4 ? 2 * ((pl.per + NWAVE - 1) / NWAVE) : (pl.per + NWAVE - 1) / NWAVE;
-    const void* fn = fmt == FMT_BF16 ? pv_pick_r<FMT_BF16>(mb, p.pv_r, pl.nld)
-                     : fmt == FMT_F16 ? pv_pick_r<FMT_F16>(mb, p.pv_r, pl.nld)
-                                      : pv_pick_r<FMT_Q4>(mb, p.pv_r, pl.nld);
+    const int pg = pv_pages(pl.nbuf);
+    SKV_CHECK(pg == 1 ? pl.nld >= 4 : pl.nld <= 4, "decode: P @ V plan of %d copies and %d buffers", pl.nld, pl.nbuf);
+    const void* fn = fmt == FMT_BF16 ? pv_pick_r<FMT_BF16>(mb, p.pv_r, pl.nld, pg)
+                     : fmt == FMT_F16 ? pv_pick_r<FMT_F16>(mb, p.pv_r, pl.nld, pg)
+                                      : pv_pick_r<FMT_Q4>(mb, p.pv_r, pl.nld, pg);
     int rc = raise_lds(fn, PV_MAX_DYN_LDS);
     if (rc) return rc;
     void* args[] = {(void*)&a};
