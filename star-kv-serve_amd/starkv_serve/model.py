@@ -308,7 +308,7 @@ class StarKVLlamaForCausalLM:
         if md.num_decodes or not md.num_prefills:
             raise ValueError("prefill_step: a prompts-only batch (prefill_metadata)")
         x = self._layers(self.embed[tokens], positions, md, capture, False)
-        last = torch.tensor(md.prefill_query_start_loc_cpu[1:], device=x.device) - 1
+        last = torch.tensor([e - 1 for e in md.prefill_query_start_loc_cpu[1:]]).to(x.device, non_blocking=True)
         return self._logits(x[last], False)
 
 
