@@ -715,7 +715,8 @@ __global__ __launch_bounds__(LIFT_THR) void lift_kernel(const uint8_t* __restric
 // LDS and come back transposed (ds_read_b64_tr_b16); B = the rows o as three bf16 values each (8 + 8
 // + 8 bits hold an fp32 value exactly, so the products are those of fp32 o and their sums fp32: no
 // less precise than fmaf, where an inf or NaN takes the first value only). The vector form spends 8
-// fmaf and an LDS read per 8 columns and request. LIFT_FIGURES
+// fmaf and an LDS read per 8 columns and request: 64 requests of r_v 1290 21.8 us against 14.1, 24 of
+// r_v 1280 18.3 against 11.2.
 constexpr int LM_WAVES = 8;
 constexpr int LM_BATCH = 6;  // steps of 32 rank columns in flight per wave
 constexpr int LM_LDS = LM_WAVES * LM_BATCH * 2048;

@@ -19,7 +19,10 @@ def _rows_ok(t: torch.Tensor) -> bool:
 
 
 def rope_fits(cos_sin: torch.Tensor, positions: torch.Tensor, *rows: torch.Tensor) -> bool:
-    """Whether the kernel takes these rows (q, and k and v): GPU tensors of one dtype."""
+    """Whether the kernel takes these rows (q, and k and v): GPU tensors of one dtype, no gradient
+    wanted."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in rows):
+        return False
     return (all(t.is_cuda and t.dtype == rows[0].dtype and t.dtype in _FLOATS and _rows_ok(t) for t in rows)
             and cos_sin.device == positions.device == rows[0].device and cos_sin.dtype in _FLOATS
             and cos_sin.dim() == 2 and cos_sin.shape[1] == 128 and cos_sin.is_contiguous()
