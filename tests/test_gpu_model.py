@@ -247,3 +247,36 @@ def test_stock_decode_splits_of_larger_batches(cuda, lens):
             truth[i, h] = torch.softmax(K[:, h] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, h]
     assert_close(out[live], truth.cpu().numpy(), f"stock splits n={n}")
     assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
+
+
+@pytest.mark.parametrize("Hkv", [4, 2])
+@pytest.mark.parametrize("shape", ["rising", "falling", "jumps", "flat"])
+def test_gqa_decode_moves_its_reference_max(cuda, Hkv, shape):
+    """Two query heads a row, with scores that pass the reference max by more than 2^8 slowly, never,
+    or from page to page (the last page partly filled). Against float64: bf16 output (half an ulp is at
+    most 2^-8 of the value); a float32 score of up to 100 over 128 terms is off by at most 100 * 8 * 2^-24
+    = 5e-5, and so are the weights, times |V| < 5."""
+    g = torch.Generator().manual_seed(Hkv)
+    Hq, bs, lens = 8, 16, [1003, 70, 16]
+    pages = [(L + bs - 1) // bs for L in lens]
+    nb = sum(pages) + 1
+    kc, vc = (torch.randn(nb, bs, Hkv, 128, generator=g).to(torch.bfloat16) for _ in range(2))
+    vc.clamp_(-4.5, 4.5)
+    q = torch.randn(len(lens), Hq, 128, generator=g).to(torch.bfloat16)
+    q[..., 0] = 8
+    bt, o = torch.zeros(len(lens), max(pages), dtype=torch.int32), 1
+    for b, p in enumerate(pages):
+        bt[b, :p] = torch.arange(o, o + p)
+        ramp = {"rising": torch.linspace(0, 60, p * bs), "falling": torch.linspace(60, 0, p * bs),
+                "jumps": (60 * torch.rand(p, generator=g)).repeat_interleave(bs), "flat": torch.zeros(p * bs)}[shape]
+        kc[o:o + p, :, :, 0] = ramp.view(p, bs, 1).to(torch.bfloat16)
+        o += p
+    out = paged_decode_full(q.to(cuda), kc.to(cuda), vc.to(cuda), bt.to(cuda),
+                            torch.tensor(lens, dtype=torch.int32, device=cuda), max(lens), 128 ** -0.5).double().cpu()
+    for b, L in enumerate(lens):
+        K, V = (t[bt[b, :pages[b]].long()].reshape(-1, Hkv, 128)[:L].double() for t in (kc, vc))
+        for h in range(Hq):
+            kv = h // (Hq // Hkv)
+            want = torch.softmax(K[:, kv] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, kv]
+            err = (out[b, h] - want).abs() - want.abs() * 2 ** -8
+            assert err.max() < 2.5e-4, (shape, b, h, float(err.max()))
