@@ -5,6 +5,7 @@ starkv_serve/model.py:77-106 there)."""
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from starkv_serve import _hip
 
@@ -18,10 +19,18 @@ def _rows_ok(t: torch.Tensor) -> bool:
             and t.stride(1) % step == 0 and t.data_ptr() % 16 == 0)
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """Not a subclass (a tracer's tensor), a transform's wrapper (vmap, jvp) or a dual tensor."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and forward_ad.unpack_dual(t).tangent is None)
+
+
 def rope_fits(cos_sin: torch.Tensor, positions: torch.Tensor, *rows: torch.Tensor) -> bool:
     """Whether the kernel takes these rows (q, and k and v): GPU tensors of one dtype, no gradient
-    wanted."""
+    wanted in either direction, not traced or mapped."""
     if torch.is_grad_enabled() and any(t.requires_grad for t in rows):
+        return False
+    if not all(_plain(t) for t in (cos_sin, positions, *rows)):
         return False
     return (all(t.is_cuda and t.dtype == rows[0].dtype and t.dtype in _FLOATS and _rows_ok(t) for t in rows)
             and cos_sin.device == positions.device == rows[0].device and cos_sin.dtype in _FLOATS

@@ -115,3 +115,25 @@ def test_few_linear(cuda, n, N, K, dt):
     s = F.silu(a)
     check(mo.few_linear(x, w, nw, 1e-5, gate=True), s * b,
           1.1 * err[:, :N] * (b.abs() + err[:, N:]) + s.abs() * err[:, N:] + (s * b).abs() * 2.0 ** -20)
+
+
+def test_rotary_under_transforms(cuda):
+    """vmap, jvp, dual tensors and gradients through Rotary.apply take torch's operations: the plain
+    call's values, and the rotation of the tangent (it is linear in x)."""
+    from starkv_serve.model import Rotary
+    g = torch.Generator().manual_seed(3)
+    rot = Rotary(50, torch.float32, cuda, 10000.0)
+    pos = torch.tensor([0, 49, 7], device=cuda)
+    x, dx = (torch.randn(2, 3, 4, 128, generator=g).to(cuda) for _ in range(2))
+    want, dwant = ([rot.apply(pos, t[i]) for i in range(2)] for t in (x, dx))
+    near = lambda a, b: torch.testing.assert_close(a, b, rtol=0, atol=8 * 8 * 2 ** -24)  # |x| < 8, up to 8 fp32 roundings
+    near(torch.vmap(lambda t: rot.apply(pos, t))(x), torch.stack(want))
+    out, tan = torch.func.jvp(lambda t: rot.apply(pos, t), (x[0],), (dx[0],))
+    near(out, want[0])
+    near(tan, dwant[0])
+    with torch.autograd.forward_ad.dual_level():
+        dual = rot.apply(pos, torch.autograd.forward_ad.make_dual(x[0], dx[0]))
+        near(torch.autograd.forward_ad.unpack_dual(dual).tangent, dwant[0])
+    leaf = x[0].clone().requires_grad_()
+    (rot.apply(pos, leaf) * want[0]).sum().backward()  # the rotation's transpose undoes it
+    near(leaf.grad, x[0])
