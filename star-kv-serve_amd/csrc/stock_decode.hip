@@ -35,6 +35,7 @@ struct StockParams {
     const int32_t* bt; int64_t bt_s0, bt_s1;
     const int32_t* seq_lens;
     int n, Hq, Hkv, max_seq_len, splits, pps;  // pps: pages per split
+    int R;                                     // workgroups per (request, split, KV head)
     float sc;                                  // scale * log2(e)
     float* part;                               // [n][Hq][splits][2 + 128]
     void* out; int64_t o_s0, o_s1; int out_dt;
@@ -67,8 +68,17 @@ template <int CDT, int G>
 __global__ __launch_bounds__(ST_THR) void stock_decode_kernel(const StockParams p) {
     __shared__ float s_m[4][G], s_l[4][G];
     __shared__ float s_acc[4][G][128];
-    const int s = blockIdx.x, b = blockIdx.z;
-    const int hq0 = blockIdx.y * G;                 // the workgroup's first query head
+    int s = blockIdx.x, b = blockIdx.z;
+    int hq0 = blockIdx.y * G;                       // the workgroup's first query head
+    if (G > 1 && p.R > 1) {
+        // Workgroup id: runs of 8 units (request, split, KV head), R times each, so that the R
+        // workgroups of a unit are 8 ids apart: on one XCD, at one time.
+        const int id = blockIdx.x, u = id / (8 * p.R) * 8 + id % 8;
+        if (u >= p.n * p.splits * p.Hkv) return;
+        b = u / (p.splits * p.Hkv);
+        s = u / p.Hkv % p.splits;
+        hq0 = (u % p.Hkv * p.R + id / 8 % p.R) * G;
+    }
     const int h = hq0 / (p.Hq / p.Hkv);             // its KV head
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int t = lane >> 2, c = lane & 3;
@@ -289,8 +299,8 @@ const void* stock_pick(int gw) {
 
 // Splits per (request, head group): enough workgroups to fill the device (2 per CU), at
 // least 8 pages per split, at most ST_MAX_SPLITS. groups = workgroups per request and split;
-// mha: one query head per KV head.
-int stock_splits(int n, int groups, int max_seq_len, bool mha) {
+// group: query heads per KV head.
+int stock_splits(int n, int groups, int max_seq_len, int group) {
     const int pages = (max_seq_len + 15) / 16;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -313,7 +323,22 @@ int stock_splits(int n, int groups, int max_seq_len, bool mha) {
     // 324, 24 x 3072 280 against 248, 64 x 4096 806 / 536 against 780 / 501. Whole rounds of short
     // requests stay as they are: 16 x 3072 169 / 131 against 174 / 133, 64 x 2048 422 / 292 against
     // 414 / 299.
-    if (mha && wgs > cus && pages >= 192 && (wgs % (2 * cus) != 0 || pages >= 256)) s = wgs < 2 * cus ? 5 : 3;
+    if (group == 1 && wgs > cus && pages >= 192 && (wgs % (2 * cus) != 0 || pages >= 256)) s = wgs < 2 * cus ? 5 : 3;
+    // Four or eight query heads per KV head, whose workgroups read K and V from their XCD's L2 and are
+    // bound by their instructions: the split count with the least rounds of the device times a
+    // round's pages and about 30 pages of start and end, of the most that fit one round and 1, 3 and 5
+    // (odd for the reason above: 48 x 1024 to 8192 349 us with one, 389 with two, 314 with three). 8 KV
+    // heads, the count that just passes a round / this one, us: 10 x 8192 142 / 110, 12 x 8192
+    // 180 / 142, 20 x 8192 253 / 207, 24 x 8192 281 / 260, ragged 235 / 190, 48 x 8192 508 / 463, 24 x
+    // 3000 119 / 107.
+    if (group > 2) {
+        const int64_t slots = 2 * (int64_t)cus, most = (pages + 7) / 8;
+        const auto cost = [&](int64_t k) { return (wgs * k + slots - 1) / slots * ((pages + k - 1) / k + 30); };
+        int64_t best = std::max<int64_t>(1, std::min<int64_t>({slots / wgs, most, ST_MAX_SPLITS}));
+        for (const int64_t k : {1, 3, 5})
+            if (k <= most && cost(k) < cost(best)) best = k;
+        s = (int)best;
+    }
     s = std::min(s, ST_MAX_SPLITS);
     return s < 1 ? 1 : s;
 }
@@ -329,7 +354,7 @@ extern "C" {
 size_t starkv_stock_decode_workspace_bytes(int n, int num_heads, int num_kv_heads, int max_seq_len) {
     if (n < 1 || num_heads < 1 || num_kv_heads < 1 || max_seq_len < 1) return 0;
     const int splits = stock_splits(n, num_heads == num_kv_heads ? num_heads : num_heads / 2, max_seq_len,
-                                    num_heads == num_kv_heads);
+                                    num_heads / num_kv_heads);
     return splits == 1 ? 256 : (size_t)n * num_heads * splits * 130 * 4;
 }
 
@@ -360,7 +385,7 @@ int starkv_stock_decode(void* stream, const void* query, int64_t q_s0, int64_t q
     SKV_CHECK(q_s0 % 8 == 0 && q_s1 % 8 == 0 && ((uintptr_t)query % 16) == 0,
               "stock_decode: query rows must be 16-byte aligned");
     const int gw = G == 1 ? 1 : 2;
-    const int splits = stock_splits(n, num_heads / gw, max_seq_len, gw == 1);
+    const int splits = stock_splits(n, num_heads / gw, max_seq_len, G);
     const size_t need = starkv_stock_decode_workspace_bytes(n, num_heads, num_kv_heads, max_seq_len);
     SKV_CHECK(workspace_bytes >= need, "stock_decode: workspace %zu bytes < %zu", workspace_bytes, need);
     StockParams p;
@@ -370,12 +395,14 @@ int starkv_stock_decode(void* stream, const void* query, int64_t q_s0, int64_t q
     p.bt = block_table; p.bt_s0 = bt_s0; p.bt_s1 = bt_s1; p.seq_lens = seq_lens;
     p.n = n; p.Hq = num_heads; p.Hkv = num_kv_heads; p.max_seq_len = max_seq_len; p.splits = splits;
     p.pps = ((max_seq_len + 15) / 16 + splits - 1) / splits;
+    p.R = G / gw;
     p.sc = scale * ST_LOG2E;
     p.part = (float*)workspace;
     p.out = out; p.o_s0 = o_s0; p.o_s1 = o_s1; p.out_dt = out_dtype;
     const void* fn = cache_dtype == STARKV_BF16 ? stock_pick<STARKV_BF16>(gw) : stock_pick<STARKV_F16>(gw);
     void* args[] = {(void*)&p};
-    SKV_HIP(hipLaunchKernel(fn, dim3(splits, num_heads / gw, n), dim3(ST_THR), args, 0, (hipStream_t)stream));
+    const dim3 grid = p.R > 1 ? dim3((n * splits * num_kv_heads + 7) / 8 * 8 * p.R) : dim3(splits, num_heads / gw, n);
+    SKV_HIP(hipLaunchKernel(fn, grid, dim3(ST_THR), args, 0, (hipStream_t)stream));
     if (splits > 1) {
         hipLaunchKernelGGL(stock_merge_kernel, dim3(num_heads, n), dim3(128), 0, (hipStream_t)stream, p);
         SKV_HIP(hipGetLastError());

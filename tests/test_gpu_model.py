@@ -280,3 +280,32 @@ def test_gqa_decode_moves_its_reference_max(cuda, Hkv, shape):
             want = torch.softmax(K[:, kv] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, kv]
             err = (out[b, h] - want).abs() - want.abs() * 2 ** -8
             assert err.max() < 2.5e-4, (shape, b, h, float(err.max()))
+
+
+@pytest.mark.parametrize("Hq,Hkv,lens", [(32, 8, [8100 - 330 * i for i in range(24)]), (32, 8, [2900] * 5 + [0, 17]),
+                                         (8, 1, [333, 1, 0]), (12, 3, [129] * 9), (32, 8, [700] * 33), (16, 2, [4097] * 33)])
+def test_gqa_decode_units_and_splits(cuda, Hq, Hkv, lens):
+    """Two or four workgroups of a (request, split, KV head), also where those are no multiple of 8:
+    1, 3, 5 and many splits, some past a request's end, empty requests (NaN). Against float64 in torch,
+    by the decode tolerance."""
+    g = torch.Generator().manual_seed(len(lens))
+    bs, n = 16, len(lens)
+    pages = [(L + bs - 1) // bs for L in lens]
+    nb = sum(pages) + 1
+    kc, vc = (torch.randn(nb, bs, Hkv, 128, generator=g).to(torch.bfloat16).to(cuda) for _ in range(2))
+    bt, o = torch.zeros(n, max(pages), dtype=torch.int32), 1
+    for b, p in enumerate(pages):
+        bt[b, :p] = torch.arange(o, o + p)
+        o += p
+    q = torch.randn(n, Hq, 128, generator=g).to(torch.bfloat16).to(cuda)
+    out = paged_decode_full(q, kc, vc, bt.to(cuda), torch.tensor(lens, dtype=torch.int32, device=cuda), max(lens),
+                            128 ** -0.5)
+    live = [b for b in range(n) if lens[b]]
+    truth = torch.empty(len(live), Hq, 128, dtype=torch.float64, device=cuda)
+    for i, b in enumerate(live):
+        K, V = (t[bt[b, :pages[b]].long().to(cuda)].reshape(-1, Hkv, 128)[:lens[b]].double() for t in (kc, vc))
+        for h in range(Hq):
+            kv = h // (Hq // Hkv)
+            truth[i, h] = torch.softmax(K[:, kv] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, kv]
+    assert_close(out[live], truth.cpu().numpy(), f"GQA units Hq={Hq} Hkv={Hkv} n={n}")
+    assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
