@@ -22,11 +22,12 @@ __device__ __forceinline__ int64_t load_slot(const void* slots, int bits, int i)
 
 // clamp(rint(x / s)) + 8 with the division rounded once. |x| <= 7 s in a block, so the product with
 // the approximate reciprocal is within 2^-18 of the quotient: 2^-17 and more away from a midpoint
-// it rounds to the same integer, and only else (or for inf and NaN) is the division made.
+// it rounds to the same integer, and only else (or for inf and NaN) is the division made. So is it
+// where s > 2^126, whose reciprocal is subnormal: the approximation gives 0 there.
 __device__ __forceinline__ int quant_code(float x, float s, float lo, float hi) {
     const float y = x * __builtin_amdgcn_rcpf(s);
     float q = rintf(y);
-    if (!(fabsf(y - q) < 0.5f - 0x1p-17f)) q = rintf(__fdiv_rn(x, s));
+    if (!(fabsf(y - q) < 0.5f - 0x1p-17f && s <= 0x1p126f)) q = rintf(__fdiv_rn(x, s));
     q = fminf(fmaxf(q, lo), hi);
     return (int)(q + 8.0f);
 }

@@ -155,3 +155,27 @@ def test_pack_kv_rows_too_long_for_lds_and_lanes_no_head_holds(cuda):
         pq.pack_kv(k.to(cuda), v.to(cuda), cache, slots.to(cuda), row, i32(ranks), i32(offsets), i32(nouts))
         end = row.vq_off + row.v_bytes
         assert np.array_equal(cache.cpu().numpy()[:, :, :end], want[:, :, :end])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_pack_kv_scales_past_2_126(cuda, dtype):
+    """Codes near the largest finite values: an inlier block's scale (its maximum / 3) has a subnormal
+    reciprocal. Every byte as the CPU packer's, whose division has no such edge."""
+    ranks, R = [16, 32], 40
+    widths, offsets, W = ref.head_layout(ranks)
+    nouts = [ref.n_outlier(r) for r in ranks]
+    row = pq.QuantRow(W, len(ranks), R)
+    g = torch.Generator().manual_seed(9)
+    k, v = (torch.rand(6, w, generator=g) * 2 - 1 for w in (W, R))
+    top = torch.tensor([3.3e38, 2.6e38, 2.5e38, 1e38, 3e38, 1.0])[:, None]  # inlier scales on both sides of 2^126
+    k, v = (k * top).to(dtype), (v * top).to(dtype)
+    k[:, -1], v[:, -1] = top[:, 0].to(dtype), -top[:, 0].to(dtype)
+    slots = torch.arange(16, 22)
+    want = np.zeros((2, 16, row.nbytes), np.uint8)
+    cquant.pack_kv(k.float().numpy(), v.float().numpy(), want, slots.numpy(), ranks, offsets, nouts, R, row.ks_off,
+                   row.vs_off, row.vq_off)
+    cache = torch.zeros(2, 16, row.nbytes, dtype=torch.uint8, device=cuda)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=cuda)  # noqa: E731
+    pq.pack_kv(k.to(cuda), v.to(cuda), cache, slots.to(cuda), row, i32(ranks), i32(offsets), i32(nouts))
+    assert (want[1, 0, row.vq_off:] >> 4).max() > 8  # codes that are not 0
+    assert np.array_equal(cache.cpu().numpy(), want)
