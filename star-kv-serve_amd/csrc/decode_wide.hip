@@ -714,9 +714,10 @@ __global__ __launch_bounds__(LIFT_THR) void lift_kernel(const uint8_t* __restric
 // steps of 32 of them in flight. A = v_up^T: a step's 32 rows x 64 bytes go through the wave's own
 // LDS and come back transposed (ds_read_b64_tr_b16); B = the rows o as three bf16 values each (8 + 8
 // + 8 bits hold an fp32 value exactly, so the products are those of fp32 o and their sums fp32: no
-// less precise than fmaf, where an inf or NaN takes the first value only). The vector form spends 8
-// fmaf and an LDS read per 8 columns and request: 64 requests of r_v 1290 21.8 us against 14.1, 24 of
-// r_v 1280 18.3 against 11.2.
+// less precise than fmaf, where an inf or NaN takes the first value only). An infinite weight meets
+// the zero among the three values: a result that is not finite is formed again by fmaf over the
+// rows. The vector form spends 8 fmaf and an LDS read per 8 columns and request: 64 requests of
+// r_v 1290 21.8 us against 14.1, 24 of r_v 1280 18.3 against 11.2.
 constexpr int LM_WAVES = 8;
 constexpr int LM_BATCH = 6;  // steps of 32 rank columns in flight per wave
 constexpr int LM_LDS = LM_WAVES * LM_BATCH * 2048;
@@ -834,6 +835,12 @@ __global__ __launch_bounds__(64 * LM_WAVES) void lift_matrix_kernel(const uint8_
 #pragma unroll
         for (int k = 0; k < LM_WAVES; ++k)
             v += ((const float*)&sum[((k * RT + t) * 2 + (col >> 4)) * 64 + 16 * ((col >> 2) & 3) + r])[col & 3];
+        if (!(fabsf(v) < INFINITY)) {
+            const float* o = (const float*)(ws + ws_o) + ((int64_t)b * Hq + h) * ld;
+            const uint16_t* wc = vup + (int64_t)h * vu_s0 + d0 + col;
+            v = 0.f;
+            for (int k = 0; k < v_rank && v == v; ++k) v = fmaf(o[k], bf16_bits_to_f32(wc[(int64_t)k * vu_s1]), v);
+        }
         store_f(out, (int64_t)b * o_s0 + (int64_t)h * o_s1 + d0 + col, out_dt, v);
     }
 }

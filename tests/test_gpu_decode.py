@@ -587,3 +587,28 @@ def test_two_pass_lift_on_matrix_instructions(cuda, n, v_rank, quant):
     # Averages of normal codes: |o| <= 8. Two fp32 sums of v_rank products each.
     bound = 2 * v_rank * 2.0 ** -24 * 8 * v16.double().abs().sum(1).max()
     assert ((a - b).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("n", [5, 17])
+def test_two_pass_lift_of_infinite_weights(cuda, n):
+    """An infinite or NaN weight of v_up_by_q, one to a head: the fp32 sum over the rank columns, inf by its sign
+    where the column's merged value is not 0, as the vector form (fp16 weights of the same values)."""
+    lens = [0] + [17 + 29 * i for i in range(n - 1)]
+    g = W.make_lowrank(lens, num_heads=8, seed=n, v_rank=1288).to(cuda)
+    args = list(g.decode_args())
+    at = [i for i, a in enumerate(args) if torch.is_tensor(a) and a.data_ptr() == g.v_up_by_q.data_ptr()][0]
+    vu = g.v_up_by_q.to(torch.float16).to(torch.bfloat16)
+    vu[0, 3, 7], vu[1, 1283, 127], vu[2, 640, 31], vu[3, 5, 32] = float("inf"), -float("inf"), float("nan"), float("inf")
+    vu[3, 6, 32] = float("inf")
+    outs = []
+    for dt in (torch.bfloat16, torch.float16):
+        args[at] = vu.to(dt)
+        out = torch.empty(n, 8, 128, dtype=torch.float32, device=cuda)
+        paged_starkv_decode(*args, out=out)
+        outs.append(out)
+    a, b = outs[0][1:], outs[1][1:]
+    assert outs[0][0].isnan().all()
+    assert b[:, 0, 7].isinf().all() and b[:, 1, 127].isinf().all() and b[:, 2, 31].isnan().all()
+    odd = ~torch.isfinite(b)
+    assert odd.sum() == 4 * (n - 1) and torch.equal(~torch.isfinite(a), odd)
+    assert torch.equal(a[odd].nan_to_num(nan=7.0), b[odd].nan_to_num(nan=7.0))
