@@ -81,6 +81,14 @@ def greedy_step(logits: torch.Tensor, tokens: torch.Tensor, positions: torch.Ten
     _hip.ops().greedy_step(logits, tokens, positions)
 
 
+def few_fits(*tensors: torch.Tensor) -> bool:
+    """Whether ``few_linear`` takes these operands (rows, weights, the norm's weight, the residual): no
+    gradient wanted in either direction, not traced or mapped."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return all(_plain(t) for t in tensors)
+
+
 def few_linear(x: torch.Tensor, w: torch.Tensor, norm_weight: Optional[torch.Tensor] = None, eps: float = 0.0,
                h_out: Optional[torch.Tensor] = None, gate: bool = False,
                residual: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -214,16 +214,16 @@ class StarKVLlamaForCausalLM:
     def _norm_linear(self, x: torch.Tensor, ln: torch.Tensor, w: torch.Tensor, few: bool, want_h: bool) -> tuple:
         """(the normalised x, when wanted, its product with w)."""
         s = self.shape
-        if few and self.dtype == torch.bfloat16:
+        if few and self.dtype == torch.bfloat16 and model_ops.few_fits(x, w, ln):
             h = torch.empty_like(x) if want_h else None
             return h, model_ops.few_linear(x, w, ln, s.rms_norm_eps, h)
         h = F.rms_norm(x, (s.hidden_size,), ln, s.rms_norm_eps)
-        return h, model_ops.few_linear(h, w) if few else F.linear(h, w)
+        return h, model_ops.few_linear(h, w) if few and model_ops.few_fits(h, w) else F.linear(h, w)
 
     def _mlp(self, x: torch.Tensor, layer: Layer, few: bool) -> torch.Tensor:
         """x plus the gated MLP of its norm."""
         s = self.shape
-        if few and self.dtype == torch.bfloat16:
+        if few and self.dtype == torch.bfloat16 and model_ops.few_fits(x, layer.gate_up, layer.ln2):
             a = model_ops.few_linear(x, layer.gate_up, layer.ln2, s.rms_norm_eps, gate=True)
         else:
             gu = self._norm_linear(x, layer.ln2, layer.gate_up, few, False)[1]
@@ -236,7 +236,7 @@ class StarKVLlamaForCausalLM:
 
     @staticmethod
     def _add_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, few: bool) -> torch.Tensor:
-        return model_ops.few_linear(a, w, residual=x) if few else x + F.linear(a, w)
+        return model_ops.few_linear(a, w, residual=x) if few and model_ops.few_fits(a, w, x) else x + F.linear(a, w)
 
     @torch.no_grad()
     def attention_inputs(self, hidden: torch.Tensor, positions: torch.Tensor) -> List[tuple]:

@@ -309,3 +309,26 @@ def test_gqa_decode_units_and_splits(cuda, Hq, Hkv, lens):
             truth[i, h] = torch.softmax(K[:, kv] @ q[b, h].double() * 128 ** -0.5, 0) @ V[:, kv]
     assert_close(out[live], truth.cpu().numpy(), f"GQA units Hq={Hq} Hkv={Hkv} n={n}")
     assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_decode_logits_are_differentiable(cuda, dtype):
+    """decode_step's logits carry a gradient to the norm and the head where one is wanted (the layers run
+    without): bit for bit the values and gradients of torch's norm and product of the same rows."""
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, dtype=dtype, seed=2)
+    model.allocate_kv_cache(9)
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    pos = torch.tensor([3, 0], device=cuda)
+    tokens = torch.tensor([5, 6], device=cuda)
+    x = model._layers(model.embed[tokens], pos, M.decode_metadata(bt, pos, 16, 4), None, False)
+    leaves = [t.clone().requires_grad_() for t in (model.norm, model.lm_head)]
+    want = torch.nn.functional.linear(torch.nn.functional.rms_norm(x, (SHAPE.hidden_size,), leaves[0],
+                                                                   SHAPE.rms_norm_eps), leaves[1])
+    model.norm.requires_grad_()
+    model.lm_head.requires_grad_()
+    logits = model.decode_step(tokens, pos, M.decode_metadata(bt, pos, 16, 4))
+    assert torch.equal(logits, want)
+    logits.float().square().sum().backward()
+    want.float().square().sum().backward()
+    for got, leaf in zip((model.norm, model.lm_head), leaves):
+        assert torch.equal(got.grad, leaf.grad)
