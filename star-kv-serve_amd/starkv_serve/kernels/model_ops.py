@@ -81,12 +81,17 @@ def greedy_step(logits: torch.Tensor, tokens: torch.Tensor, positions: torch.Ten
     _hip.ops().greedy_step(logits, tokens, positions)
 
 
-def few_fits(*tensors: torch.Tensor) -> bool:
-    """Whether ``few_linear`` takes these operands (rows, weights, the norm's weight, the residual): no
-    gradient wanted in either direction, not traced or mapped."""
+def few_fits(x: torch.Tensor, w: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
+             residual: Optional[torch.Tensor] = None) -> bool:
+    """Whether ``few_linear`` takes these operands: rows that 16-byte loads can take, K a multiple of a matrix
+    step, no gradient wanted in either direction, not traced or mapped."""
+    tensors = [t for t in (x, w, norm_weight, residual) if t is not None]
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    return all(_plain(t) for t in tensors)
+    return (all(_plain(t) and t.stride(-1) == 1 and t.dtype == x.dtype for t in tensors)
+            and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w))
+            and (norm_weight is None or norm_weight.data_ptr() % 16 == 0)
+            and bool(_hip.lib().starkv_few_linear_fits(x.shape[0], x.shape[1])))
 
 
 def few_linear(x: torch.Tensor, w: torch.Tensor, norm_weight: Optional[torch.Tensor] = None, eps: float = 0.0,

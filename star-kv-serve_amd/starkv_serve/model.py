@@ -206,10 +206,8 @@ class StarKVLlamaForCausalLM:
         where the weights' bytes are the time. Llama-2-7B's widths at 16 tokens, us, against the
         library's products with torch's norm, gate and sum: q 14 / 21, qkv 35 / 35, o 12 / 18, gate and
         up 53 / 67, down 30 / 41, the head 74 / 68; the kernel's matrix tile holds 16 tokens."""
-        s = self.shape
         return (self.device.type == "cuda" and not md.num_prefills and 1 <= T <= FEW_MAX_TOKENS
-                and self.dtype in (torch.bfloat16, torch.float16) and s.hidden_size % 32 == 0
-                and s.intermediate_size % 32 == 0)
+                and self.dtype in (torch.bfloat16, torch.float16))
 
     def _norm_linear(self, x: torch.Tensor, ln: torch.Tensor, w: torch.Tensor, few: bool, want_h: bool) -> tuple:
         """(the normalised x, when wanted, its product with w)."""
@@ -236,7 +234,7 @@ class StarKVLlamaForCausalLM:
 
     @staticmethod
     def _add_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, few: bool) -> torch.Tensor:
-        return model_ops.few_linear(a, w, residual=x) if few and model_ops.few_fits(a, w, x) else x + F.linear(a, w)
+        return model_ops.few_linear(a, w, residual=x) if few and model_ops.few_fits(a, w, residual=x) else x + F.linear(a, w)
 
     @torch.no_grad()
     def attention_inputs(self, hidden: torch.Tensor, positions: torch.Tensor) -> List[tuple]:

@@ -332,3 +332,30 @@ def test_decode_logits_are_differentiable(cuda, dtype):
     want.float().square().sum().backward()
     for got, leaf in zip((model.norm, model.lm_head), leaves):
         assert torch.equal(got.grad, leaf.grad)
+
+
+def test_decode_step_takes_weights_in_any_layout(cuda):
+    """Weights as transposed views, and at starts and row strides that no wide load can take: torch's products,
+    within bf16's rounding of the contiguous weights' logits."""
+    shape = M.LlamaShape(hidden_size=512, num_layers=2, num_heads=4, num_kv_heads=2, head_dim=128,
+                         intermediate_size=1024, vocab_size=999)
+    model = M.StarKVLlamaForCausalLM(shape, None, max_model_len=64, device=cuda, seed=3)
+    model.allocate_kv_cache(9)
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    pos = torch.tensor([0, 0], device=cuda)
+    step = lambda: model.decode_step(torch.tensor([1, 2], device=cuda), pos, M.decode_metadata(bt, pos, 16, 1))  # noqa: E731
+    want = step()
+
+    def odd(t):  # the same values, 2 bytes off, rows 2 bytes longer
+        return torch.cat([t.new_zeros(1), torch.nn.functional.pad(t, (0, 1)).reshape(-1)])[1:].view(
+            t.shape[0], -1)[:, :t.shape[1]]
+
+    for layout in (odd, lambda t: t.t().contiguous().t()):
+        for layer in model.layers:
+            layer.qkv_proj, layer.o_proj, layer.gate_up, layer.down = map(
+                layout, (layer.qkv_proj, layer.o_proj, layer.gate_up, layer.down))
+        model.lm_head = layout(model.lm_head)
+        got = step()
+        rel = (got.double() - want.double()).norm() / want.double().norm()
+        # A dozen roundings of 2^-9 (rms about 2^-9 / sqrt(3)) on the way, either side.
+        assert rel < 2 * 12 * 2.0 ** -9, float(rel)
