@@ -180,7 +180,7 @@ class StarKVLlamaForCausalLM:
             layer.impl.forward_from_hidden(q.view(T, H * D), h, self.kv_caches[li], md, out, in_full_graph=in_graph)
         else:
             h, qkv = self._norm_linear(x, layer.ln1, layer.qkv_proj, few, capture is not None)
-            q, k, v = (t.view(T, -1, D) for t in qkv.split([H * D, Hkv * D, Hkv * D], dim=-1))
+            q, k, v = (t.view(T, n, D) for t, n in zip(qkv.split([H * D, Hkv * D, Hkv * D], dim=-1), (H, Hkv, Hkv)))
             kc, vc = self.kv_caches[li]
             ka, va = k, v  # the prefill attention's operands
             if model_ops.rope_fits(self.rotary.cos_sin_cache, positions, q, k, v):

@@ -359,3 +359,12 @@ def test_decode_step_takes_weights_in_any_layout(cuda):
         rel = (got.double() - want.double()).norm() / want.double().norm()
         # A dozen roundings of 2^-9 (rms about 2^-9 / sqrt(3)) on the way, either side.
         assert rel < 2 * 12 * 2.0 ** -9, float(rel)
+
+
+def test_decode_step_of_no_tokens(cuda):
+    """A step without requests: empty logits, through uncompressed layers."""
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, seed=2)
+    model.allocate_kv_cache(2)
+    none = torch.zeros(0, dtype=torch.int64, device=cuda)
+    bt = torch.zeros(0, 4, dtype=torch.int32, device=cuda)
+    assert model.decode_step(none, none, M.decode_metadata(bt, none, 16, 1)).shape == (0, SHAPE.vocab_size)
