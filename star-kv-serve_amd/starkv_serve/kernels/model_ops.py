@@ -8,6 +8,7 @@ import torch
 from torch.autograd import forward_ad
 
 from starkv_serve import _hip
+from starkv_serve.kernels.paged_decode import _as_i32
 
 _FLOATS = (torch.bfloat16, torch.float16, torch.float32)
 
@@ -55,8 +56,8 @@ def rope_write(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
     q_out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     k_out = torch.empty(k.shape, dtype=k.dtype, device=k.device) if keep_k else None
     kv16 = torch.empty((2, *k.shape), dtype=torch.float16, device=k.device) if half else (None, None)
-    _hip.ops().rope_qkv(q, k, v, positions, cos_sin, q_out, k_out, k_cache, v_cache, slots.contiguous(), kv16[0],
-                        kv16[1])
+    slots = slots.contiguous() if slots.dtype == torch.int64 else _as_i32(slots)
+    _hip.ops().rope_qkv(q, k, v, positions, cos_sin, q_out, k_out, k_cache, v_cache, slots, kv16[0], kv16[1])
     return q_out, k_out, kv16[0], kv16[1]
 
 

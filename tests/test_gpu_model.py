@@ -368,3 +368,15 @@ def test_decode_step_of_no_tokens(cuda):
     none = torch.zeros(0, dtype=torch.int64, device=cuda)
     bt = torch.zeros(0, 4, dtype=torch.int32, device=cuda)
     assert model.decode_step(none, none, M.decode_metadata(bt, none, 16, 1)).shape == (0, SHAPE.vocab_size)
+
+
+def test_decode_step_takes_other_slot_types(cuda):
+    """Slots of an integer type the write has no form for are converted, as write_kv_full does."""
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, seed=2)
+    model.allocate_kv_cache(9)
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    pos, tokens = torch.tensor([0, 0], device=cuda), torch.tensor([1, 2], device=cuda)
+    md = M.decode_metadata(bt, pos, 16, 1)
+    want = model.decode_step(tokens, pos, md)
+    md.slot_mapping = md.slot_mapping.to(torch.int16)
+    assert torch.equal(model.decode_step(tokens, pos, md), want)
