@@ -34,7 +34,7 @@ def rope_fits(cos_sin: torch.Tensor, positions: torch.Tensor, *rows: torch.Tenso
     if not all(_plain(t) for t in (cos_sin, positions, *rows)):
         return False
     return (all(t.is_cuda and t.dtype == rows[0].dtype and t.dtype in _FLOATS and _rows_ok(t) for t in rows)
-            and cos_sin.device == positions.device == rows[0].device and cos_sin.dtype in _FLOATS
+            and all(t.device == rows[0].device for t in (cos_sin, positions, *rows)) and cos_sin.dtype in _FLOATS
             and cos_sin.dim() == 2 and cos_sin.shape[1] == 128 and cos_sin.is_contiguous()
             and cos_sin.data_ptr() % 16 == 0 and positions.dim() == 1 and positions.is_contiguous()
             and positions.dtype in (torch.int32, torch.int64) and positions.numel() == rows[0].shape[0])
@@ -46,6 +46,19 @@ def rope(positions: torch.Tensor, x: torch.Tensor, cos_sin: torch.Tensor) -> tor
     if x.numel():
         _hip.ops().rope_qkv(x, None, None, positions, cos_sin, out, None, None, None, None, None, None)
     return out
+
+
+def rope_write_fits(cos_sin: torch.Tensor, positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                    k_cache: torch.Tensor, v_cache: torch.Tensor, slots: torch.Tensor) -> bool:
+    """Whether ``rope_write`` may stand for the rotations and ``write_kv_full``: rows the kernel takes, and caches
+    and slots that write_kv_full accepts (it refuses the others itself)."""
+    bs = k_cache.shape[1]
+    return (all(t.device == q.device for t in (k_cache, v_cache, slots))
+            and k_cache.dtype == v_cache.dtype == q.dtype and q.dtype in (torch.bfloat16, torch.float16)
+            and k_cache.shape == v_cache.shape and k_cache.shape[2:] == k.shape[1:] == v.shape[1:]
+            and k_cache.stride() == v_cache.stride() and k_cache.stride(-1) == 1
+            and all(s % 8 == 0 for s in k_cache.stride()[:3]) and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
+            and bs >= 16 and bs & (bs - 1) == 0 and rope_fits(cos_sin, positions, q, k, v))
 
 
 def rope_write(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos_sin: torch.Tensor,
@@ -84,12 +97,12 @@ def greedy_step(logits: torch.Tensor, tokens: torch.Tensor, positions: torch.Ten
 
 def few_fits(x: torch.Tensor, w: torch.Tensor, norm_weight: Optional[torch.Tensor] = None,
              residual: Optional[torch.Tensor] = None) -> bool:
-    """Whether ``few_linear`` takes these operands: rows that 16-byte loads can take, K a multiple of a matrix
+    """Whether ``few_linear`` takes these operands, on one device: rows that 16-byte loads can take, K a multiple of a matrix
     step, no gradient wanted in either direction, not traced or mapped."""
     tensors = [t for t in (x, w, norm_weight, residual) if t is not None]
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    return (all(_plain(t) and t.stride(-1) == 1 and t.dtype == x.dtype for t in tensors)
+    return (all(t.device == x.device and _plain(t) and t.stride(-1) == 1 and t.dtype == x.dtype for t in tensors)
             and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w))
             and (norm_weight is None or norm_weight.data_ptr() % 16 == 0)
             and bool(_hip.lib().starkv_few_linear_fits(x.shape[0], x.shape[1])))

@@ -183,13 +183,14 @@ class StarKVLlamaForCausalLM:
             q, k, v = (t.view(T, n, D) for t, n in zip(qkv.split([H * D, Hkv * D, Hkv * D], dim=-1), (H, Hkv, Hkv)))
             kc, vc = self.kv_caches[li]
             ka, va = k, v  # the prefill attention's operands
-            if model_ops.rope_fits(self.rotary.cos_sin_cache, positions, q, k, v):
-                q, k, ka, va = model_ops.rope_write(positions, q, k, v, self.rotary.cos_sin_cache, kc, vc,
-                                                    md.slot_mapping[:T], capture is not None, bool(md.num_prefills))
+            slots = md.slot_mapping[:T]
+            if model_ops.rope_write_fits(self.rotary.cos_sin_cache, positions, q, k, v, kc, vc, slots):
+                q, k, ka, va = model_ops.rope_write(positions, q, k, v, self.rotary.cos_sin_cache, kc, vc, slots,
+                                                    capture is not None, bool(md.num_prefills))
             else:
                 q, k = self.rotary.apply(positions, q), self.rotary.apply(positions, k)
                 ka = k
-                write_kv_full(k, v, kc, vc, md.slot_mapping[:T])
+                write_kv_full(k, v, kc, vc, slots)
             if md.num_prefills:  # whole prompts only (prefill_step): causal attention over each prompt
                 out = prefill_attention(q, ka, va, md.prefill_seq_lens_cpu, self.scale).view(T, H * D)
             else:

@@ -380,3 +380,28 @@ def test_decode_step_takes_other_slot_types(cuda):
     want = model.decode_step(tokens, pos, md)
     md.slot_mapping = md.slot_mapping.to(torch.int16)
     assert torch.equal(model.decode_step(tokens, pos, md), want)
+
+
+def test_steps_refuse_caches_the_write_refuses(cuda):
+    """Caches on the host, of another type, with different strides, of a block size the decode has no form for:
+    write_kv_full's errors, nothing launched on them; a weight on the host: torch's."""
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, seed=2)
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    pos, tokens = torch.tensor([0, 0], device=cuda), torch.tensor([1, 2], device=cuda)
+    md = M.decode_metadata(bt, pos, 16, 1)
+    pmd, ppos = M.prefill_metadata(bt, [1, 1], 16)
+    good = torch.zeros(9, 16, 4, 128, dtype=torch.bfloat16, device=cuda)
+    wide = torch.zeros(9, 16, 8, 128, dtype=torch.bfloat16, device=cuda)[:, :, :4]
+    for kc, vc in ((good.cpu(), good.cpu()), (good, good.cpu()), (good.float(), good.float()), (good, wide),
+                   (good[:, :12], good[:, :12])):
+        model.kv_caches = [(kc, vc)] * SHAPE.num_layers
+        for step in (lambda: model.decode_step(tokens, pos, md), lambda: model.prefill_step(tokens, ppos, pmd)):
+            with pytest.raises((RuntimeError, AssertionError)):
+                step()
+    model.kv_caches = [(good, good.clone()) for _ in range(SHAPE.num_layers)]
+    want = model.decode_step(tokens, pos, md)
+    model.lm_head = model.lm_head.cpu()
+    with pytest.raises(RuntimeError):
+        model.decode_step(tokens, pos, md)
+    model.lm_head = model.lm_head.to(cuda)
+    assert torch.equal(model.decode_step(tokens, pos, md), want)

@@ -2,6 +2,7 @@
 import torch
 
 from starkv_serve import model as M
+from starkv_serve.kernels import model_ops
 
 
 def test_decode_step_of_no_tokens():
@@ -13,3 +14,16 @@ def test_decode_step_of_no_tokens():
     none = torch.zeros(0, dtype=torch.int64)
     bt = torch.zeros(0, 4, dtype=torch.int32)
     assert model.decode_step(none, none, M.decode_metadata(bt, none, 16, 1)).shape == (0, 10)
+
+
+def test_kernels_are_not_given_memory_of_another_device():
+    """Weights, caches or slots beside the step's own device go to the calls that refuse them."""
+    bf = dict(dtype=torch.bfloat16)
+    x, w, ln = (torch.zeros(*s, device="meta", **bf) for s in ((2, 64), (32, 64), (64,)))
+    assert model_ops.few_fits(x, w, ln)
+    assert not model_ops.few_fits(x, torch.zeros(32, 64, **bf), ln)
+    assert not model_ops.few_fits(x, w, torch.zeros(64, **bf))
+    q, k, cs = (torch.zeros(*s, device="meta", **bf) for s in ((2, 4, 128), (2, 2, 128), (9, 128)))
+    kc, pos, slots = torch.zeros(3, 16, 2, 128, **bf), torch.zeros(2, device="meta").long(), torch.zeros(2).long()
+    for a in ((kc, kc, slots), (kc.to("meta"), kc, slots.to("meta")), (kc.to("meta"), kc.to("meta"), slots)):
+        assert not model_ops.rope_write_fits(cs, pos, q, k, k, *a)
