@@ -429,14 +429,15 @@ int starkv_prefill_lift(void *stream, const void *k_codes, int64_t k_s0, const v
  *
  * starkv_rope_qkv: rotate-half RoPE of q [T, num_heads, 128] and, when given, k [T, num_kv_heads,
  * 128] at positions [T] (int32 or int64; a negative one counts from the table's end, one outside
- * it gives NaN) of cos_sin [cs_rows, 128] = cos | sin: fp32 arithmetic, rounded once to the inputs'
- * dtype (bf16, fp16 or fp32). q_out and k_out are contiguous; k_cache / v_cache [num_blocks,
+ * it ends the launch with a device error, as torch's index does) of cos_sin [cs_rows, 128] = cos |
+ * sin: fp32 arithmetic, rounded once to the inputs' dtype (bf16, fp16 or fp32). q_out and k_out are contiguous; k_cache / v_cache [num_blocks,
  * block_size, num_kv_heads, 128] (shared element strides) take the rotated k and v at slot_mapping
  * (a slot outside the cache: nothing); k_half / v_half [T, num_kv_heads, 128] take them in fp16.
  * Every destination but q_out may be null. All rows 16-byte aligned.
  *
  * starkv_decode_slots: slots[b] = block_table[b][positions[b] / block_size] * block_size +
- * positions[b] % block_size (-1 outside the row of `width` blocks) and seq_lens[b] = positions[b] + 1.
+ * positions[b] % block_size and seq_lens[b] = positions[b] + 1; a block outside the row of `width`
+ * entries (negative ones count from its end) ends the launch with a device error.
  *
  * starkv_greedy_step: tokens[b] = the index of the first largest of logits [n, width] (bf16, fp16 or
  * fp32, rows 16-byte aligned; NaN counts as the largest), positions[b] += 1.

@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "decode_pages.hpp"
+#include "index_rules.hpp"
 
 namespace starkv {
 
@@ -91,15 +92,10 @@ __global__ __launch_bounds__(256) void rope_qkv_kernel(const RopeParams p) {
     load8_f(src, at + 64 + d, p.dt, b);
     if (!isv) {
         int64_t pos = p.pos64 ? ((const int64_t*)p.pos)[t] : (int64_t)((const int32_t*)p.pos)[t];
-        if (pos < 0) pos += p.cs_rows;  // as an index counts from the end
+        if (!wrap_index(pos, p.cs_rows)) __builtin_trap();
         float c[8], s[8];
-        if (pos >= 0 && pos < p.cs_rows) {
-            load8_f(p.cs, pos * p.cs_s0 + d, p.cs_dt, c);
-            load8_f(p.cs, pos * p.cs_s0 + 64 + d, p.cs_dt, s);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) c[e] = s[e] = __builtin_nanf("");
-        }
+        load8_f(p.cs, pos * p.cs_s0 + d, p.cs_dt, c);
+        load8_f(p.cs, pos * p.cs_s0 + 64 + d, p.cs_dt, s);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float2 r = rotate(a[e], b[e], c[e], s[e]);
@@ -134,7 +130,7 @@ __global__ __launch_bounds__(256) void rope_qkv_kernel(const RopeParams p) {
 // ---------------------------------------------------------------------------
 // A decode step's slots and lengths from its positions: one launch for what took ten of torch's
 // on a step's critical path. A block index counts from the row's end when negative, as an index
-// does; one outside the row gives slot -1.
+// does; one outside the row ends the launch.
 // ---------------------------------------------------------------------------
 template <typename BT>
 __global__ __launch_bounds__(256) void decode_slots_kernel(const BT* __restrict__ bt, int64_t s0, int64_t s1, int width,
@@ -143,13 +139,9 @@ __global__ __launch_bounds__(256) void decode_slots_kernel(const BT* __restrict_
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= n) return;
     const int64_t p = pos[b];
-    int64_t blk = p / block_size, in = p % block_size;
-    if (in < 0) {
-        in += block_size;
-        --blk;
-    }
-    if (blk < 0) blk += width;
-    slots[b] = blk >= 0 && blk < width ? (int64_t)bt[b * s0 + blk * s1] * block_size + in : -1;
+    int64_t blk, in;
+    if (!split_position(p, block_size, width, blk, in)) __builtin_trap();
+    slots[b] = (int64_t)bt[b * s0 + blk * s1] * block_size + in;
     lens[b] = (int32_t)(p + 1);
 }
 

@@ -1,4 +1,8 @@
 """Host logic of the model's steps that needs no GPU."""
+import ctypes
+import os
+import subprocess
+
 import torch
 
 from starkv_serve import model as M
@@ -27,3 +31,35 @@ def test_kernels_are_not_given_memory_of_another_device():
     kc, pos, slots = torch.zeros(3, 16, 2, 128, **bf), torch.zeros(2, device="meta").long(), torch.zeros(2).long()
     for a in ((kc, kc, slots), (kc.to("meta"), kc, slots.to("meta")), (kc.to("meta"), kc.to("meta"), slots)):
         assert not model_ops.rope_write_fits(cs, pos, q, k, k, *a)
+
+
+def test_index_rules_are_those_of_torch(tmp_path):
+    """The positions a decode step's kernels take (csrc/index_rules.hpp, built for the host): those torch's index
+    takes, at the same places; at every other the kernels end the launch."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(M.__file__))), "csrc")
+    src, so = tmp_path / "rules.cpp", tmp_path / "rules.so"
+    src.write_text('#include "index_rules.hpp"\n'
+                   'extern "C" int wrap(int64_t* i, int64_t n) { return starkv::wrap_index(*i, n); }\n'
+                   'extern "C" int split(int64_t p, int64_t bs, int64_t w, int64_t* b, int64_t* in) '
+                   '{ return starkv::split_position(p, bs, w, *b, *in); }\n')
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", f"-I{csrc}", str(src), "-o", str(so)], check=True)
+    L, i64 = ctypes.CDLL(str(so)), ctypes.c_int64
+    table, row, bs = torch.arange(50), torch.arange(7), 16
+    for p in list(range(-130, 130)) + [2 ** 40, -2 ** 40, 2 ** 63 - 1, -2 ** 63]:
+        for rule in ("table", "row"):
+            pos, a, b = torch.tensor([p]), i64(p), i64()
+            if rule == "table":
+                ok = L.wrap(ctypes.byref(a), i64(50))
+            else:
+                ok = L.split(i64(p), i64(bs), i64(7), ctypes.byref(a), ctypes.byref(b))
+            try:
+                want = table[pos] if rule == "table" else row[pos // bs]
+            except IndexError:
+                assert not ok, (rule, p)
+                continue
+            assert ok and a.value == want.item(), (rule, p)
+            if rule == "row":
+                assert b.value == (pos % bs).item(), p
+    kernels = open(os.path.join(csrc, "model_ops.hip")).read()
+    assert kernels.count("__builtin_trap()") == 2 and "wrap_index(pos, p.cs_rows)" in kernels
+    assert "split_position(p, block_size, width, blk, in)" in kernels
