@@ -193,6 +193,23 @@ class StarKVAttentionImpl:
         # V's lift runs as an fp16 GEMM (fp32 accumulation, the result rounded once to fp16).
         self.v_up_f16 = self.w.v_up.to(device=device, dtype=torch.float16).contiguous()  # [H * Hd, v_rank]
 
+    # The padded operands of a batched K lift (attention.py:144-160): what a program of its own over the
+    # codes may read; the prompts' lift here takes heads at their own widths.
+    @property
+    def k_prefill_gather(self) -> torch.Tensor:
+        """[H * k_max_rank]: each head's code columns; lanes past a head's width point at its first."""
+        idx = [off + (r if r < width else 0)
+               for off, width in zip(self.w.k_head_offsets.tolist(), self.w.k_head_widths.tolist())
+               for r in range(self.w.k_max_rank)]
+        return torch.tensor(idx, dtype=torch.long, device=self.k_up_f32.device)
+
+    @property
+    def k_up_T(self) -> torch.Tensor:
+        """[H, k_max_rank, 128] fp32: U by head, zero in the lanes past a head's width."""
+        lanes = torch.arange(self.w.k_max_rank, device=self.k_up_f32.device)
+        up = self.k_up_f32[self.k_prefill_gather].view(self.num_kv_heads, -1, self.head_size)
+        return up.masked_fill(lanes[None, :, None] >= self.k_head_widths[:, None, None], 0.0)
+
     def _cache(self, kv_cache: torch.Tensor) -> torch.Tensor:
         cache = kv_cache.squeeze(1) if kv_cache.dim() == 4 else kv_cache  # [num_blocks, block_size, width]
         return cache if self.row is None else cache.view(torch.uint8)

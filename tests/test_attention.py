@@ -69,6 +69,19 @@ def test_to_device_operands(layers, quant):
         assert impl.row.nbytes % 16 == 0 and impl.k_nouts.numel() == 4
 
 
+def test_padded_lift_operands(layers):
+    """codes[:, k_prefill_gather] in heads of k_max_rank times k_up_T: every head's own product."""
+    w = layers[0]
+    impl = _impl(w)
+    impl.to_device(torch.device("cpu"), torch.bfloat16)
+    H, R = impl.num_kv_heads, w.k_max_rank
+    assert impl.k_up_T.shape == (H, R, 128) and impl.k_up_T.dtype == torch.float32
+    codes = torch.randint(-4, 5, (3, w.k_width)).float()
+    got = torch.bmm(codes[:, impl.k_prefill_gather].view(3, H, R).transpose(0, 1).contiguous(), impl.k_up_T)
+    for h, (o, n) in enumerate(zip(w.k_head_offsets.tolist(), w.k_head_widths.tolist())):
+        torch.testing.assert_close(got[h], codes[:, o:o + n] @ w.k_up[o:o + n].float())
+
+
 def _md(n_dec, n_pre, prompt=1, cached=0):
     """n_dec decodes, then n_pre prompts of `prompt` tokens each with `cached` tokens of
     context already in the cache."""
