@@ -6,6 +6,7 @@ from typing import Optional
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 from starkv_serve import _hip
 from starkv_serve.kernels.paged_decode import _as_i32
@@ -20,6 +21,12 @@ def _rows_ok(t: torch.Tensor) -> bool:
             and t.stride(1) % step == 0 and t.data_ptr() % 16 == 0)
 
 
+def _traced() -> bool:
+    """Under torch.compile (which cannot look into ``_plain``), torch.jit.trace or a dispatch mode (make_fx, fake
+    tensors): what is recorded there are torch's operations."""
+    return torch.compiler.is_compiling() or torch.jit.is_tracing() or is_in_torch_dispatch_mode()
+
+
 def _plain(t: torch.Tensor) -> bool:
     """Not a subclass (a tracer's tensor), a transform's wrapper (vmap, jvp) or a dual tensor."""
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
@@ -29,7 +36,7 @@ def _plain(t: torch.Tensor) -> bool:
 def rope_fits(cos_sin: torch.Tensor, positions: torch.Tensor, *rows: torch.Tensor) -> bool:
     """Whether the kernel takes these rows (q, and k and v): GPU tensors of one dtype, no gradient
     wanted in either direction, not traced or mapped."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in rows):
+    if _traced() or (torch.is_grad_enabled() and any(t.requires_grad for t in rows)):
         return False
     if not all(_plain(t) for t in (cos_sin, positions, *rows)):
         return False
@@ -82,6 +89,14 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def slots_fit(block_table: torch.Tensor, positions: torch.Tensor) -> bool:
+    """Whether ``decode_slots`` takes this step: GPU tensors of a decode step's types, not traced or mapped."""
+    return (not _traced() and positions.is_cuda and block_table.device == positions.device
+            and positions.dtype == torch.int64 and positions.is_contiguous()
+            and block_table.dtype in (torch.int32, torch.int64) and block_table.shape[0] >= positions.shape[0]
+            and _plain(positions) and _plain(block_table))
+
+
 def decode_slots(block_table: torch.Tensor, positions: torch.Tensor, block_size: int) -> tuple:
     """(slot_mapping int64, seq_lens int32) of a decode step at `positions` [n] int64."""
     slots = torch.empty_like(positions)
@@ -100,7 +115,7 @@ def few_fits(x: torch.Tensor, w: torch.Tensor, norm_weight: Optional[torch.Tenso
     """Whether ``few_linear`` takes these operands, on one device: rows that 16-byte loads can take, K a multiple of a matrix
     step, no gradient wanted in either direction, not traced or mapped."""
     tensors = [t for t in (x, w, norm_weight, residual) if t is not None]
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    if _traced() or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
         return False
     return (all(t.device == x.device and _plain(t) and t.stride(-1) == 1 and t.dtype == x.dtype for t in tensors)
             and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w))

@@ -361,9 +361,7 @@ def decode_metadata(block_table: torch.Tensor, positions: torch.Tensor, block_si
     if max_seq_len > block_table.shape[1] * block_size:
         raise ValueError(f"positions up to {max_seq_len - 1} need more than the block table's "
                          f"{block_table.shape[1]} blocks of {block_size}")
-    if (positions.is_cuda and block_table.device == positions.device and positions.dtype == torch.int64
-            and positions.is_contiguous() and block_table.dtype in (torch.int32, torch.int64)
-            and block_table.shape[0] >= n):
+    if model_ops.slots_fit(block_table, positions):
         slots, seq_lens = model_ops.decode_slots(block_table, positions, block_size)
     else:
         rows = torch.arange(n, device=positions.device)

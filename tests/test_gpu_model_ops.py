@@ -137,3 +137,27 @@ def test_rotary_under_transforms(cuda):
     leaf = x[0].clone().requires_grad_()
     (rot.apply(pos, leaf) * want[0]).sum().backward()  # the rotation's transpose undoes it
     near(leaf.grad, x[0])
+
+
+def test_rotary_and_slots_compile_and_trace(cuda):
+    """torch.compile (one graph), jit.trace and make_fx of Rotary.apply and torch.compile of decode_metadata see torch's
+    operations only, and give the plain calls' values."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from starkv_serve.model import Rotary, decode_metadata
+    g = torch.Generator().manual_seed(3)
+    rot = Rotary(50, torch.float32, cuda, 10000.0)
+    pos = torch.tensor([0, 49, 7], device=cuda)
+    x = torch.randn(3, 4, 128, generator=g).to(cuda)
+    want = rot.apply(pos, x)
+    near = lambda a, b: torch.testing.assert_close(a, b, rtol=0, atol=8 * 8 * 2 ** -24)  # as above
+    near(torch.compile(rot.apply, fullgraph=True, backend="eager")(pos, x), want)
+    traced = torch.jit.trace(rot.apply, (pos, x), check_trace=False)
+    assert "starkv::" not in str(traced.graph)
+    near(traced(pos[:2], x[:2]), want[:2])
+    bt = torch.arange(12, dtype=torch.int32, device=cuda).view(3, 4)
+    graph = make_fx(lambda p, t: rot.apply(p, t))(pos, x)
+    assert "starkv." not in graph.code
+    near(graph(pos, x), want)
+    md, got = (f(bt, pos, 16, 64) for f in (decode_metadata, torch.compile(decode_metadata, fullgraph=True,
+                                                                          backend="eager")))
+    assert torch.equal(md.slot_mapping, got.slot_mapping) and torch.equal(md.seq_lens, got.seq_lens)

@@ -3,7 +3,9 @@ import ctypes
 import os
 import subprocess
 
+import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from starkv_serve import model as M
 from starkv_serve.kernels import model_ops
@@ -63,3 +65,21 @@ def test_index_rules_are_those_of_torch(tmp_path):
     kernels = open(os.path.join(csrc, "model_ops.hip")).read()
     assert kernels.count("__builtin_trap()") == 2 and "wrap_index(pos, p.cs_rows)" in kernels
     assert "split_position(p, block_size, width, blk, in)" in kernels
+
+
+@pytest.mark.parametrize("how", ["compile", "jit", "make_fx"])
+def test_rotary_and_slots_compile_and_trace(how):
+    """One graph, of torch's operations, with the plain calls' values."""
+    rot = M.Rotary(50, torch.float32, "cpu", 10000.0)
+    pos, x = torch.tensor([0, 49, 7]), torch.randn(3, 4, 128)
+    bt = torch.arange(12, dtype=torch.int32).view(3, 4)
+
+    def slots(bt, pos):
+        md = M.decode_metadata(bt, pos, 16, 64)
+        return md.slot_mapping, md.seq_lens
+
+    for f, args in ((lambda p, t: rot.apply(p, t), (pos, x)), (slots, (bt, pos))):
+        g = {"compile": lambda: torch.compile(f, fullgraph=True, backend="eager"),
+             "jit": lambda: torch.jit.trace(f, args, check_trace=False), "make_fx": lambda: make_fx(f)(*args)}[how]()
+        got, want = g(*args), f(*args)
+        assert all(torch.equal(a, b) for a, b in zip(*((t if isinstance(t, tuple) else (t,)) for t in (got, want))))
