@@ -39,7 +39,41 @@ struct StockParams {
     float sc;                                  // scale * log2(e)
     float* part;                               // [n][Hq][splits][2 + 128]
     void* out; int64_t o_s0, o_s1; int out_dt;
+    int own;                                   // StockSplits
 };
+
+// The splits of request b that hold pages, at least one.
+__device__ __forceinline__ int stock_own_splits(const StockParams& p, int b) {
+    const int pages = (min(max(p.seq_lens[b], 0), p.max_seq_len) + 15) >> 4;
+    return max(1, (pages + p.pps - 1) / p.pps);
+}
+
+// Where requests have splits of their own: workgroup id as (request, query head, split), request by
+// request, head by head, of the splits that hold pages; the ids past them have none (false).
+__device__ __forceinline__ bool stock_own_unit(const StockParams& p, int id, int& b, int& hq, int& s, int& splits) {
+    const int lane = threadIdx.x & 63;
+    for (int b0 = 0; b0 < p.n; b0 += 64) {
+        const int own = b0 + lane < p.n ? stock_own_splits(p, b0 + lane) : 0;
+        int end = own;  // of the lane's request, in units of Hq workgroups: an inclusive scan
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(end, o, 64);
+            if (lane >= o) end += x;
+        }
+        const int total = __builtin_amdgcn_readlane(end, 63) * p.Hq;
+        if (id < total) {
+            const int at = __builtin_popcountll(__builtin_amdgcn_ballot_w64(end * p.Hq <= id));
+            splits = __builtin_amdgcn_readlane(own, at);
+            const int u = id - (__builtin_amdgcn_readlane(end, at) - splits) * p.Hq;
+            b = b0 + at;
+            hq = u / splits;
+            s = u % splits;
+            return true;
+        }
+        id -= total;
+    }
+    return false;
+}
 
 template <int CDT>
 __device__ __forceinline__ void cvt8(const uint4& w, float* o) {
@@ -70,6 +104,8 @@ __global__ __launch_bounds__(ST_THR) void stock_decode_kernel(const StockParams 
     __shared__ float s_acc[4][G][128];
     int s = blockIdx.x, b = blockIdx.z;
     int hq0 = blockIdx.y * G;                       // the workgroup's first query head
+    int splits = p.splits;
+    if (G == 1 && p.own && !stock_own_unit(p, blockIdx.x, b, hq0, s, splits)) return;
     if (G > 1 && p.R > 1) {
         // Workgroup id: runs of 8 units (request, split, KV head), R times each, so that the R
         // workgroups of a unit are 8 ids apart: on one XCD, at one time.
@@ -84,7 +120,8 @@ __global__ __launch_bounds__(ST_THR) void stock_decode_kernel(const StockParams 
     const int t = lane >> 2, c = lane & 3;
     const int L = min(max(p.seq_lens[b], 0), p.max_seq_len);
     const int pages = (L + 15) >> 4;
-    const int k0 = s * p.pps, k1 = min(k0 + p.pps, pages);
+    const int pps = G == 1 && p.own ? (pages + splits - 1) / splits : p.pps;
+    const int k0 = s * pps, k1 = min(k0 + pps, pages);
 
     float qv[G][32];
 #pragma unroll
@@ -217,7 +254,7 @@ __global__ __launch_bounds__(ST_THR) void stock_decode_kernel(const StockParams 
             a = fmaf(s_acc[w][g][d], e, a);
         }
         const int hq = hq0 + g;
-        if (p.splits == 1) {
+        if (splits == 1) {
             store_f(p.out, (int64_t)b * p.o_s0 + (int64_t)hq * p.o_s1 + d, p.out_dt, a / lt);  // L = 0: NaN
         } else {
             float* pp = p.part + (((int64_t)b * p.Hq + hq) * p.splits + s) * 130;
@@ -237,9 +274,11 @@ __global__ __launch_bounds__(128) void stock_merge_kernel(const StockParams p) {
     __shared__ float s_e[ST_MAX_SPLITS];
     __shared__ float s_red[2][2];  // per wave: max, then weighted sum
     const int hq = blockIdx.x, b = blockIdx.y, d = threadIdx.x, w = d >> 6;
+    const int splits = p.own ? stock_own_splits(p, b) : p.splits;
+    if (splits == 1) return;  // its workgroups wrote the result
     const float* pp = p.part + ((int64_t)b * p.Hq + hq) * p.splits * 130;
-    const float ms = d < p.splits ? pp[d * 130] : -INFINITY;
-    const float ls = d < p.splits ? pp[d * 130 + 1] : 0.f;
+    const float ms = d < splits ? pp[d * 130] : -INFINITY;
+    const float ls = d < splits ? pp[d * 130 + 1] : 0.f;
     const float mw = wave_max(ms);
     if ((d & 63) == 0) s_red[w][0] = mw;
     __syncthreads();
@@ -247,19 +286,19 @@ __global__ __launch_bounds__(128) void stock_merge_kernel(const StockParams p) {
     const float e = ms == -INFINITY ? 0.f : exp2f(ms - M);
     const float lw = wave_sum(ls * e);
     if ((d & 63) == 0) s_red[w][1] = lw;
-    if (d < p.splits) s_e[d] = e;
+    if (d < splits) s_e[d] = e;
     __syncthreads();
     const float lt = s_red[0][1] + s_red[1][1];
     float a = 0.f;
     int s = 0;
-    for (; s + 8 <= p.splits; s += 8) {
+    for (; s + 8 <= splits; s += 8) {
         float v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) v[u] = pp[(s + u) * 130 + 2 + d];
 #pragma unroll
         for (int u = 0; u < 8; ++u) a = fmaf(v[u], s_e[s + u], a);
     }
-    for (; s < p.splits; ++s) a = fmaf(pp[s * 130 + 2 + d], s_e[s], a);
+    for (; s < splits; ++s) a = fmaf(pp[s * 130 + 2 + d], s_e[s], a);
     store_f(p.out, (int64_t)b * p.o_s0 + (int64_t)hq * p.o_s1 + d, p.out_dt, a / lt);
 }
 
@@ -297,10 +336,15 @@ const void* stock_pick(int gw) {
     return gw == 1 ? (const void*)&stock_decode_kernel<CDT, 1> : (const void*)&stock_decode_kernel<CDT, 2>;
 }
 
+struct StockSplits {
+    int splits;  // workgroups per (request, head group)
+    bool own;    // only those that hold pages of the request
+};
+
 // Splits per (request, head group): enough workgroups to fill the device (2 per CU), at
 // least 8 pages per split, at most ST_MAX_SPLITS. groups = workgroups per request and split;
 // group: query heads per KV head.
-int stock_splits(int n, int groups, int max_seq_len, int group) {
+StockSplits stock_splits(int n, int groups, int max_seq_len, int group) {
     const int pages = (max_seq_len + 15) / 16;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -314,16 +358,20 @@ int stock_splits(int n, int groups, int max_seq_len, int group) {
     // 57.4 us with the grid sized for three).
     int s = (int)std::min<int64_t>((2 * (int64_t)cus + wgs - 1) / wgs, (int64_t)(pages + 7) / 8);
     // More than one workgroup a CU and long requests, one query head per KV head (the kernel that
-    // waits for memory): 3 splits, or 5 where the heads alone are less than a round, so that a round
-    // is less of the whole and a batch's longest requests are not one workgroup's work a head. Odd
-    // counts: workgroups are dealt to the XCDs by split first, and with an even count an XCD sees
-    // the same splits only, of which a short request's later ones are empty. One split against 3
-    // (5), us, equal lengths / ragged: 9 x 8192 305 / 210 against (239 / 171), 12 x 8192 354 / 274
-    // against (319 / 209), 16 x 8192 415 / 294 against 411 / 267, 20 x 8192 662 / 409 against 486 /
-    // 324, 24 x 3072 280 against 248, 64 x 4096 806 / 536 against 780 / 501. Whole rounds of short
-    // requests stay as they are: 16 x 3072 169 / 131 against 174 / 133, 64 x 2048 422 / 292 against
-    // 414 / 299.
-    if (group == 1 && wgs > cus && pages >= 192 && (wgs % (2 * cus) != 0 || pages >= 256)) s = wgs < 2 * cus ? 5 : 3;
+    // waits for memory): up to 3 splits a request, or 5 where the heads alone are less than a round, so
+    // that a round is less of the whole and a batch's longest requests are not one workgroup's work a
+    // head. Each request has as many of a span's third (or fifth) as its own pages fill, of equal length
+    // (the XCDs take workgroups in turn: a long and a short split by turns would be uneven), and the
+    // workgroups past the last come last: a captured step's span is far longer than its requests, and
+    // empty workgroups among the others left CUs with two of the full ones. One split by the span, these
+    // rules, us, equal lengths / 1/8 of the span to all of it / 500 tokens / 2000 tokens of the span: 9 x
+    // 8192 299 / 161 / 37 / 122, 233 / 131 / 26 / 109; 12 x 4096 183 / 126 / 41 / 152, 167 / 95 / 28 / 97;
+    // 16 x 8192 392 / 241 / 29 / 109, 394 / 198 / 32 / 111; 24 x 8192 691 / 307 / 45 / 183, 600 / 276 / 49 / 187;
+    // 64 x 4096 797 / 438 / 121 / 403, 779 / 397 / 125 / 423. Whole rounds of shorter spans keep one split:
+    // 16 x 4096 equal lengths 201 against 208.
+    const int least = wgs % (2 * cus) != 0 ? 192 : wgs > 2 * cus ? 256 : 320;
+    const bool own = group == 1 && wgs > cus && wgs < (1 << 20) && pages >= least;
+    if (own) s = wgs < 2 * cus ? 5 : 3;
     // Four or eight query heads per KV head, whose workgroups read K and V from their XCD's L2 and are
     // bound by their instructions: the split count with the least rounds of the device times a
     // round's pages and about 30 pages of start and end, of the most that fit one round and 1, 3 and 5
@@ -339,8 +387,7 @@ int stock_splits(int n, int groups, int max_seq_len, int group) {
             if (k <= most && cost(k) < cost(best)) best = k;
         s = (int)best;
     }
-    s = std::min(s, ST_MAX_SPLITS);
-    return s < 1 ? 1 : s;
+    return {std::max(1, std::min(s, ST_MAX_SPLITS)), own};
 }
 
 }  // namespace
@@ -354,7 +401,7 @@ extern "C" {
 size_t starkv_stock_decode_workspace_bytes(int n, int num_heads, int num_kv_heads, int max_seq_len) {
     if (n < 1 || num_heads < 1 || num_kv_heads < 1 || max_seq_len < 1) return 0;
     const int splits = stock_splits(n, num_heads == num_kv_heads ? num_heads : num_heads / 2, max_seq_len,
-                                    num_heads / num_kv_heads);
+                                    num_heads / num_kv_heads).splits;
     return splits == 1 ? 256 : (size_t)n * num_heads * splits * 130 * 4;
 }
 
@@ -385,7 +432,8 @@ int starkv_stock_decode(void* stream, const void* query, int64_t q_s0, int64_t q
     SKV_CHECK(q_s0 % 8 == 0 && q_s1 % 8 == 0 && ((uintptr_t)query % 16) == 0,
               "stock_decode: query rows must be 16-byte aligned");
     const int gw = G == 1 ? 1 : 2;
-    const int splits = stock_splits(n, num_heads / gw, max_seq_len, G);
+    const StockSplits sp = stock_splits(n, num_heads / gw, max_seq_len, G);
+    const int splits = sp.splits;
     const size_t need = starkv_stock_decode_workspace_bytes(n, num_heads, num_kv_heads, max_seq_len);
     SKV_CHECK(workspace_bytes >= need, "stock_decode: workspace %zu bytes < %zu", workspace_bytes, need);
     StockParams p;
@@ -395,13 +443,15 @@ int starkv_stock_decode(void* stream, const void* query, int64_t q_s0, int64_t q
     p.bt = block_table; p.bt_s0 = bt_s0; p.bt_s1 = bt_s1; p.seq_lens = seq_lens;
     p.n = n; p.Hq = num_heads; p.Hkv = num_kv_heads; p.max_seq_len = max_seq_len; p.splits = splits;
     p.pps = ((max_seq_len + 15) / 16 + splits - 1) / splits;
+    p.own = sp.own;
     p.R = G / gw;
     p.sc = scale * ST_LOG2E;
     p.part = (float*)workspace;
     p.out = out; p.o_s0 = o_s0; p.o_s1 = o_s1; p.out_dt = out_dtype;
     const void* fn = cache_dtype == STARKV_BF16 ? stock_pick<STARKV_BF16>(gw) : stock_pick<STARKV_F16>(gw);
     void* args[] = {(void*)&p};
-    const dim3 grid = p.R > 1 ? dim3((n * splits * num_kv_heads + 7) / 8 * 8 * p.R) : dim3(splits, num_heads / gw, n);
+    const dim3 grid = p.R > 1 ? dim3((n * splits * num_kv_heads + 7) / 8 * 8 * p.R)
+                      : p.own ? dim3(n * num_heads * splits) : dim3(splits, num_heads / gw, n);
     SKV_HIP(hipLaunchKernel(fn, grid, dim3(ST_THR), args, 0, (hipStream_t)stream));
     if (splits > 1) {
         hipLaunchKernelGGL(stock_merge_kernel, dim3(num_heads, n), dim3(128), 0, (hipStream_t)stream, p);

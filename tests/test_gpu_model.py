@@ -405,3 +405,31 @@ def test_steps_refuse_caches_the_write_refuses(cuda):
         model.decode_step(tokens, pos, md)
     model.lm_head = model.lm_head.to(cuda)
     assert torch.equal(model.decode_step(tokens, pos, md), want)
+
+
+@pytest.mark.parametrize("H,span,lens", [
+    (32, 16384, [500, 0, 5000, 5461, 5462, 10922, 10923, 16384, 1, 16, 17]),  # 5 splits of 205 pages, at their edges
+    (32, 8200, [0, 2736, 2737, 5472, 5473, 8200, 700, 33] * 2),               # 3 of 171, a whole round
+    (5, 3100, [3100, 0, 5] * 23 + [620, 621, 3099]),                          # more than 64 requests
+    (8, 4096, [30] * 130 + [4096, 1400])])
+def test_stock_decode_splits_by_own_length(cuda, H, span, lens):
+    """More (request, head) pairs than CUs over a span longer than most requests: each has the splits that its pages
+    fill, some one, some none (NaN). Against float64 in torch, by the decode tolerance."""
+    g = torch.Generator().manual_seed(H)
+    bs, n = 16, len(lens)
+    pages = [(L + bs - 1) // bs for L in lens]
+    kc, vc = (torch.randn(sum(pages) + 1, bs, H, 128, generator=g).to(torch.bfloat16).to(cuda) for _ in range(2))
+    bt, o = torch.zeros(n, (span + 15) // 16, dtype=torch.int32), 1
+    for b, p in enumerate(pages):
+        bt[b, :p] = torch.arange(o, o + p)
+        o += p
+    q = torch.randn(n, H, 128, generator=g).to(torch.bfloat16).to(cuda)
+    out = paged_decode_full(q, kc, vc, bt.to(cuda), torch.tensor(lens, dtype=torch.int32, device=cuda), span, 128 ** -0.5)
+    live = [b for b in range(n) if lens[b]]
+    truth = torch.empty(len(live), H, 128, dtype=torch.float64, device=cuda)
+    for i, b in enumerate(live):
+        K, V = (t[bt[b, :pages[b]].long().to(cuda)].reshape(-1, H, 128)[:lens[b]].double() for t in (kc, vc))
+        p = torch.softmax(torch.einsum("hd,lhd->hl", q[b].double(), K) * 128 ** -0.5, -1)
+        truth[i] = torch.einsum("hl,lhd->hd", p, V)
+    assert_close(out[live], truth.cpu().numpy(), f"own splits H={H} n={n}")
+    assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
