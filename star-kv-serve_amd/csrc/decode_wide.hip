@@ -48,7 +48,12 @@ namespace starkv {
 
 namespace {
 
-constexpr int PV_MAX_DYN_LDS = 160 * 1024 - 8192;  // beside at most 8 KB of P
+constexpr int PV_LDS = 160 * 1024;               // a workgroup's, all of a CU's
+constexpr int LIFT_MAX_DYN_LDS = PV_LDS - 1024;  // of lift_kernel, whose static LDS is a few words
+
+// Copies per wave and page, at most. With so many a wave without a last chunk copies the one before
+// again, to the same place; with fewer such a copy reads nothing, into a 1 KB block past the buffers.
+constexpr int PV_NLD = 7;
 
 // Swizzled slot of token t in granule column G.
 __device__ __forceinline__ int gslot(int G, int t) { return t ^ ((G & 1) << 2); }
@@ -81,7 +86,6 @@ struct PvParams {
                      // u0 + k at LDS unit 1 + k (ng = 2 + 2 per granules copied)
     int ng_all;      // 3.2-bit: granules of V bytes in a row from v_off
     int nch;         // 1 KB chunks copied per page: logits (2), the slot's maxima (1), then V
-    int nld;         // copies per wave per page
     int nbuf;        // page buffers (2 .. 8): nbuf - 1 pages in flight
     int buf_bytes;   // LDS bytes per page buffer (nch KB)
     int lds_bytes;
@@ -121,7 +125,8 @@ constexpr int PV_V0 = 3;
 
 // The copies of this wave for one page's V (descriptor rv) into the buffer at LDS byte `buf`
 // and the logits and maxima of the page after it (rl, rm) into the buffer at `lbuf`: copy i
-// moves chunk 8 i + wave; chunks past nch go to the dummy block and read nothing.
+// moves chunk 8 i + wave; chunks past nch go to the dummy block and read nothing, or, with PV_NLD
+// copies, are the wave's chunk before (in `off` too).
 template <int NLD>
 __device__ __forceinline__ void pv_copies(const PvParams& p, const PvPage& d, uint32_t buf, uint32_t lbuf, uint32_t dummy,
                                           int wave, const uint32_t (&off)[NLD]) {
@@ -131,7 +136,9 @@ __device__ __forceinline__ void pv_copies(const PvParams& p, const PvPage& d, ui
         if (i == 0 && wave < PV_V0)
             lds_copy16(wave < 2 ? d.rl : d.rm, lbuf + (uint32_t)ch * 1024u, off[i]);
         else
-            lds_copy16(d.rv, ch < p.nch ? buf + (uint32_t)ch * 1024u : dummy, off[i]);
+            lds_copy16(d.rv, ch < p.nch     ? buf + (uint32_t)ch * 1024u
+                             : NLD < PV_NLD ? dummy
+                                            : buf + (uint32_t)(ch - NWAVE) * 1024u, off[i]);
     }
 }
 
@@ -163,13 +170,15 @@ __device__ __forceinline__ void pv_wait(int nbuf) {
         wait_vmcnt_lgkm0_wide((nbuf - 2 * PG) * NLD);
 }
 
+// LDS of P: of the current and the next PG pages as the MFMA's A operand, bf16 in a high and a low part.
+constexpr int pv_p_bytes(int fmt, int pg) { return 2 * pg * (fmt == FMT_BF16 ? 2 : 1) * 1024; }
+
 // PG: pages between barriers (2 where at least 6 buffers fit).
 template <int FMT, int MB, int NLD, bool MULTI, int PG>
 __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
     extern __shared__ __attribute__((aligned(16))) uint8_t s_pv[];
-    // P of the current and the next PG pages as the MFMA's A operand: [page][bf16: high and low
-    // parts][lane][8].
-    __shared__ __attribute__((aligned(16))) uint16_t s_p[2 * PG][FMT == FMT_BF16 ? 2 : 1][64][8];
+    __shared__ __attribute__((aligned(16))) uint16_t s_p[2 * PG][FMT == FMT_BF16 ? 2 : 1][64][8];  // [page][part][lane][8]
+    static_assert(sizeof(s_p) == pv_p_bytes(FMT, PG), "the plan's LDS");
     // The parameters by value: the page loop's fields stay in registers (this kernel has
     // the registers to spare) instead of being reloaded where they are used.
     const PvParams& p = p0;
@@ -198,7 +207,8 @@ __global__ __launch_bounds__(NTHR) void pv_kernel(const PvParams p0) {
     uint32_t off[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-        const int ch = i * NWAVE + wave;
+        int ch = i * NWAVE + wave;
+        if (NLD == PV_NLD && ch >= p.nch) ch -= NWAVE;
         uint32_t o = 0x80000000u;  // past every descriptor: no access
         if (ch < 2) {
             const int h = 16 * ch + (lane >> 2);
@@ -850,7 +860,6 @@ __global__ __launch_bounds__(64 * LM_WAVES) void lift_matrix_kernel(const uint8_
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr int PV_NLD = 12;  // copies per wave per page, at most (the plan keeps nch <= 96)
 // Page bytes in flight per workgroup the plan aims for, with at least two pages in flight.
 // A page costs about the same time whatever its width (its barrier, P and copy issue), so
 // the plan takes the fewest windows that keep this much in flight: at V rank 1280 one
@@ -858,30 +867,48 @@ constexpr int PV_NLD = 12;  // copies per wave per page, at most (the plan keeps
 // (115 KB) took 346 us.
 constexpr int PV_INFLIGHT = 64 * 1024;
 
-// Copies per wave and page: the smallest of 2, 4, 6 and 12 that holds them (a page loop with the
-// count known spends no scalar work on it: 64 x 8192, V rank 1290 3.2-bit 210 -> 192 us; copies
-// past the page's chunks read nothing).
-int pv_nld(int nld) { return nld <= 2 ? 2 : nld <= 4 ? 4 : nld <= 6 ? 6 : PV_NLD; }
+// Copies per wave and page of so many chunks: 2, 4, 6 or 7, or 0 for too many (a page loop with the
+// count known spends no scalar work on it: 64 x 8192, V rank 1290 3.2-bit 210 -> 192 us).
+int pv_nld(int nch) {
+    const int n = (nch + NWAVE - 1) / NWAVE;
+    return n <= 2 ? 2 : n <= 4 ? 4 : n <= 6 ? 6 : n == PV_NLD ? PV_NLD : 0;
+}
+// LDS beside the page buffers.
+int pv_other_lds(int fmt, int pg, int nld) { return pv_p_bytes(fmt, pg) + (nld < PV_NLD ? 1024 : 0); }
 // Pages between barriers: with 6 buffers or more two keep four further pages in flight, and a
 // barrier, its wait and the loop's scalar work come once for both: 64 x 8192, V rank 1290 3.2-bit 192 ->
 // 187 us, one request of 16384 tokens 21.5 -> 20.3.
 int pv_pages(int nbuf) { return nbuf >= 6 ? 2 : 1; }
-
-template <int FMT, bool MULTI, int NLD, int PG>
-const void* pv_pick_mb(int mb) {
-    if (mb <= 2) return (const void*)&pv_kernel<FMT, 2, NLD, MULTI, PG>;
-    if (mb <= 4) return (const void*)&pv_kernel<FMT, 4, NLD, MULTI, PG>;
-    if (mb <= 6) return (const void*)&pv_kernel<FMT, 6, NLD, MULTI, PG>;
-    return (const void*)&pv_kernel<FMT, 8, NLD, MULTI, PG>;
+// Buffers of a page of nch chunks: 8 or 6 beside two pages' P, else up to 5 beside one's.
+int pv_buffers(int fmt, int nch, int nld) {
+    const int two = std::min(8, (PV_LDS - pv_other_lds(fmt, 2, nld)) / (nch * 1024)) & ~1;
+    return two >= 6 ? two : std::min(5, (PV_LDS - pv_other_lds(fmt, 1, nld)) / (nch * 1024));
 }
 
-// Six buffers hold pages of at most 25 chunks, 4 copies a wave; fewer buffers mean more than 3.
+// The kernels that a plan can ask for: 16-bit windows of up to 13 blocks of 32 columns have 8 or 6
+// buffers and 2 copies (up to 16 chunks a page) or 4; up to 29 blocks 4 copies, up to 45 6, up to 49 7.
+// 3.2-bit windows of up to 16 KB of V keep 6 buffers or more. Null for any other.
 template <int FMT, bool MULTI>
 const void* pv_pick(int mb, int nld, int pg) {
-    if (pg == 2) return nld == 2 ? pv_pick_mb<FMT, MULTI, 2, 2>(mb) : pv_pick_mb<FMT, MULTI, 4, 2>(mb);
-    if (nld <= 4) return pv_pick_mb<FMT, MULTI, 4, 1>(mb);
-    if (nld == 6) return pv_pick_mb<FMT, MULTI, 6, 1>(mb);
-    return pv_pick_mb<FMT, MULTI, PV_NLD, 1>(mb);
+    if constexpr (FMT == FMT_Q4) {
+        if (pg == 2 && nld == 2)
+            return mb <= 2   ? (const void*)&pv_kernel<FMT, 2, 2, MULTI, 2>
+                   : mb <= 4 ? (const void*)&pv_kernel<FMT, 4, 2, MULTI, 2>
+                   : mb <= 6 ? (const void*)&pv_kernel<FMT, 6, 2, MULTI, 2>
+                   : mb <= 8 ? (const void*)&pv_kernel<FMT, 8, 2, MULTI, 2>
+                             : nullptr;
+        return pg == 2 && nld == 4 && mb <= 8 ? (const void*)&pv_kernel<FMT, 8, 4, MULTI, 2> : nullptr;
+    } else {
+        if (pg == 2 && mb <= 2)
+            return nld == 2 ? (const void*)&pv_kernel<FMT, 2, 2, MULTI, 2> : nld == 4 ? (const void*)&pv_kernel<FMT, 2, 4, MULTI, 2> : nullptr;
+        if (nld == 4 && mb <= 4)
+            return pg == 2 ? (const void*)&pv_kernel<FMT, 4, 4, MULTI, 2> : (const void*)&pv_kernel<FMT, 4, 4, MULTI, 1>;
+        if (pg == 1 && nld == 6 && mb <= 6)
+            return mb <= 4 ? (const void*)&pv_kernel<FMT, 4, 6, MULTI, 1> : (const void*)&pv_kernel<FMT, 6, 6, MULTI, 1>;
+        if (pg == 1 && nld == PV_NLD && mb <= 8)
+            return mb <= 6 ? (const void*)&pv_kernel<FMT, 6, PV_NLD, MULTI, 1> : (const void*)&pv_kernel<FMT, 8, PV_NLD, MULTI, 1>;
+        return nullptr;
+    }
 }
 
 template <int FMT>
@@ -947,10 +974,9 @@ static PvPlan pv_plan(int fmt, int v_col, int v_rank, int vs_off, int vq_off, in
         const bool q_win = fmt == FMT_Q4 && per < pl.units;
         const int ng = fmt == FMT_Q4 ? (q_win ? 2 + 2 * per : pl.ng_all) : 4 * per;
         const int nch = (ng + 3) / 4 + PV_V0;
-        if ((nch + NWAVE - 1) / NWAVE > PV_NLD) continue;
-        int nbuf = std::min(8, (PV_MAX_DYN_LDS - 1024) / (nch * 1024));
+        const int nld = pv_nld(nch);
+        const int nbuf = nld > 0 ? pv_buffers(fmt, nch, nld) : 0;
         if (nbuf < 2) continue;
-        nbuf -= nbuf % pv_pages(nbuf);
         const int inflight = (nbuf - 1) * nch * 1024;
         const int score = inflight >= PV_INFLIGHT && nbuf >= 3 ? (1 << 30) - launches : inflight;
         if (score > best_score) {
@@ -958,8 +984,8 @@ static PvPlan pv_plan(int fmt, int v_col, int v_rank, int vs_off, int vq_off, in
             pl.per = per;
             pl.nbuf = nbuf;
             pl.nch = nch;
-            pl.nld = pv_nld((nch + NWAVE - 1) / NWAVE);
-            pl.lds = nbuf * nch * 1024 + 1024;
+            pl.nld = nld;
+            pl.lds = nbuf * nch * 1024 + (nld < PV_NLD ? 1024 : 0);
             pl.ng = ng;
             pl.q_u1 = q_win ? 1 : 0;
             pl.ok = true;
@@ -986,7 +1012,7 @@ int launch_pv(const DecodeParams& p, int fmt, int grid, hipStream_t stream) {
     a.vs_rel = p.vs_off - pl.v_off;
     a.vq_rel = p.vq_off - pl.v_off;
     a.v_nout = p.v_nout; a.v_nbo = p.v_nbo;
-    a.nch = pl.nch; a.nld = pl.nld; a.nbuf = pl.nbuf; a.buf_bytes = pl.nch * 1024;
+    a.nch = pl.nch; a.nbuf = pl.nbuf; a.buf_bytes = pl.nch * 1024;
     a.lds_bytes = pl.lds;
     a.ws = p.ws; a.ws_plan = p.ws_plan; a.ws_m = p.ws_m; a.ws_acc = p.ws_acc; a.ws_lg = p.ws_lg; a.lcap = p.lcap;
     a.acc_ld = p.acc_ld;
@@ -999,11 +1025,11 @@ int launch_pv(const DecodeParams& p, int fmt, int grid, hipStream_t stream) {
     const int windows = (pl.units + pl.per - 1) / pl.per;
     const int mb = fmt == FMT_Q4 ? 2 * ((pl.per + NWAVE - 1) / NWAVE) : (pl.per + NWAVE - 1) / NWAVE;
     const int pg = pv_pages(pl.nbuf);
-    SKV_CHECK(pg == 1 ? pl.nld >= 4 : pl.nld <= 4, "decode: P @ V plan of %d copies and %d buffers", pl.nld, pl.nbuf);
     const void* fn = fmt == FMT_BF16 ? pv_pick_r<FMT_BF16>(mb, p.pv_r, pl.nld, pg)
                      : fmt == FMT_F16 ? pv_pick_r<FMT_F16>(mb, p.pv_r, pl.nld, pg)
                                       : pv_pick_r<FMT_Q4>(mb, p.pv_r, pl.nld, pg);
-    int rc = raise_lds(fn, PV_MAX_DYN_LDS);
+    SKV_CHECK(fn, "decode: no P @ V kernel of %d blocks a wave, %d copies, %d buffers", mb, pl.nld, pl.nbuf);
+    int rc = raise_lds(fn, PV_LDS - pv_p_bytes(fmt, pg));
     if (rc) return rc;
     void* args[] = {(void*)&a};
     SKV_HIP(hipLaunchKernel(fn, dim3(gp, windows), dim3(NTHR), args, (size_t)a.lds_bytes, stream));
@@ -1013,13 +1039,13 @@ int launch_pv(const DecodeParams& p, int fmt, int grid, hipStream_t stream) {
 bool pv_fits(int fmt, int k_width, int v_rank, int vs_off, int vq_off, int v_nout, int v_bytes) {
     (void)v_nout;
     return pv_plan(fmt, k_width, v_rank, vs_off, vq_off, v_bytes).ok &&
-           lift_lds((v_rank + 3) & ~3) <= (size_t)PV_MAX_DYN_LDS;
+           lift_lds((v_rank + 3) & ~3) <= (size_t)LIFT_MAX_DYN_LDS;
 }
 
 int launch_merge_wide(const DecodeParams& p, int grid, int w_dt, const void* vup, int64_t vu_s0, int64_t vu_s1,
                       void* out, int64_t o_s0, int64_t o_s1, int out_dt, hipStream_t stream) {
     const size_t lds = lift_lds(p.acc_ld);
-    SKV_CHECK(lds <= (size_t)PV_MAX_DYN_LDS, "decode: v_rank %d too large for the merge", p.v_rank);
+    SKV_CHECK(lds <= (size_t)LIFT_MAX_DYN_LDS, "decode: v_rank %d too large for the merge", p.v_rank);
     // Partials per request: about gp / n + 1, many of them split over the waves. Whole decode at W 880,
     // r_v 1280, us, with 16, 4 and 1 waves' phases: 1 request of 16384 tokens 65.7, 62.5, 72.6; 2 of 8192
     // 65.9, 62.5, 64.6; 8 of 4096 84.7, 80.6, 79.8; 24 179.5, 162.6, 159.7; 48 310, 263, 259.
@@ -1054,10 +1080,10 @@ int launch_merge_wide(const DecodeParams& p, int grid, int w_dt, const void* vup
                            : (w_dt == STARKV_BF16 ? (const void*)&lift_kernel<STARKV_BF16, 8, 512, 16>
                               : w_dt == STARKV_F16 ? (const void*)&lift_kernel<STARKV_F16, 8, 512, 16>
                                                    : (const void*)&lift_kernel<STARKV_F32, 8, 512, 16>);
-    int rc = raise_lds(fn, PV_MAX_DYN_LDS);
+    int rc = raise_lds(fn, LIFT_MAX_DYN_LDS);
     if (rc) return rc;
     const size_t lds2 = lift_lds(p.acc_ld, req, thr, dq);
-    SKV_CHECK(lds2 <= (size_t)PV_MAX_DYN_LDS, "decode: v_rank %d too large for the lift", p.v_rank);
+    SKV_CHECK(lds2 <= (size_t)LIFT_MAX_DYN_LDS, "decode: v_rank %d too large for the lift", p.v_rank);
     void* args[] = {(void*)&ws, (void*)&wo, (void*)&n, (void*)&Hq, (void*)&vr, (void*)&ld, (void*)&vup,
                     (void*)&vu_s0, (void*)&vu_s1, (void*)&out, (void*)&o_s0, (void*)&o_s1, (void*)&out_dt};
     SKV_HIP(hipLaunchKernel(fn, dim3(p.Hq, (p.n + req - 1) / req, 128 / (8 * dq)), dim3(thr), args, lds2, stream));

@@ -612,3 +612,19 @@ def test_two_pass_lift_of_infinite_weights(cuda, n):
     odd = ~torch.isfinite(b)
     assert odd.sum() == 4 * (n - 1) and torch.equal(~torch.isfinite(a), odd)
     assert torch.equal(a[odd].nan_to_num(nan=7.0), b[odd].nan_to_num(nan=7.0))
+
+
+@pytest.mark.parametrize("v_rank,dtype", [(v, torch.bfloat16) for v in (417, 481, 512, 864, 928, 929, 1121, 1441, 1505, 1537,
+                                                                       1568, 1569, 3009, 3073, 3136)]
+                         + [(v, torch.float16) for v in (481, 1121, 1537, 3136)])
+def test_two_pass_column_windows(cuda, v_rank, dtype):
+    """V ranks at the edges of the P @ V pass's plans (copies a wave, page buffers, pages a barrier, column windows) with a
+    grid of as many ranges as the device has CUs, so that the windows are as wide as they get."""
+    g = torch.Generator().manual_seed(v_rank)
+    lens = torch.randint(1, 200, (64,), generator=g).tolist()
+    wl = W.make_lowrank(lens, num_heads=4, ranks=[32, 16, 16, 32], v_rank=v_rank + (-v_rank) % 8, seed=v_rank, dtype=dtype)
+    truth = ref.lowrank_decode(wl.query.float().numpy(), wl.kv_cache.float().numpy(), wl.block_table.numpy(),
+                               wl.seq_lens.numpy(), wl.max_seq_len, wl.k_up.float().numpy(), wl.ranks,
+                               wl.k_head_offsets.tolist(), wl.k_width, wl.v_up_by_q.float().numpy(),
+                               wl.cos_sin_cache.float().numpy(), wl.scale)
+    assert_close(paged_starkv_decode(*wl.to(cuda).decode_args()), truth, f"windows of {v_rank}")
