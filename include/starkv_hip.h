@@ -35,7 +35,7 @@ extern "C" {
 #define STARKV_ERR_HIP 2
 #define STARKV_ERR_UNSUPPORTED 3
 
-/* Library ABI version (bumped on any signature change). */
+/* Library ABI version (bumped on any change of a signature and with new entry points). */
 int starkv_abi_version(void);
 
 /* Message of the last failed call on this host thread ("" if none). */

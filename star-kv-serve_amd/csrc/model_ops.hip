@@ -43,7 +43,7 @@ struct RopeParams {
     const void* q; int64_t q_s0, q_s1;  // elements; v null: q only, or q and k
     const void* k; int64_t k_s0, k_s1;
     const void* v; int64_t v_s0, v_s1;
-    int dt, H, Hkv, T;
+    int dt, H, Hkv;
     const void* pos; int pos64;
     const void* cs; int64_t cs_s0; int cs_dt; int64_t cs_rows;
     void* q_out; void* k_out;           // contiguous [T][heads][128] of the model dtype, or null
@@ -426,7 +426,7 @@ int starkv_rope_qkv(void* stream, const void* q, int64_t q_s0, int64_t q_s1, con
     p.q = q; p.q_s0 = q_s0; p.q_s1 = q_s1;
     p.k = k; p.k_s0 = k_s0; p.k_s1 = k_s1;
     p.v = v; p.v_s0 = v_s0; p.v_s1 = v_s1;
-    p.dt = dtype; p.H = num_heads; p.Hkv = num_kv_heads; p.T = num_tokens;
+    p.dt = dtype; p.H = num_heads; p.Hkv = num_kv_heads;
     p.pos = positions; p.pos64 = pos_bits == 64;
     p.cs = cos_sin; p.cs_s0 = cs_s0; p.cs_dt = cs_dtype; p.cs_rows = cs_rows;
     p.q_out = q_out; p.k_out = k_out;

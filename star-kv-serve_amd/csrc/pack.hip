@@ -242,7 +242,7 @@ using namespace starkv;
 
 extern "C" {
 
-int starkv_abi_version(void) { return 6; }
+int starkv_abi_version(void) { return 7; }
 
 const char* starkv_last_error(void) { return g_err; }
 

@@ -37,7 +37,7 @@ struct LiftParams {
     const int32_t* cu;
     const float* u; int64_t u_s0;      // [W][128]
     const int32_t* offs; const int32_t* widths;
-    const void* cs; int64_t cs_s0; int cs_dt;
+    const void* cs; int64_t cs_s0;
     uint8_t* ko;                       // fp16 [T][H][128]
     uint16_t* vo; int v_rank;          // fp16 [T][v_rank]
     int hplanes;
@@ -261,7 +261,7 @@ int starkv_prefill_lift(void* stream, const void* k_codes, int64_t k_s0, const v
     p.T = num_tokens; p.H = num_kv_heads; p.P = num_prompts;
     p.cu = cu_seqlens;
     p.u = k_up; p.u_s0 = u_s0; p.offs = k_offsets; p.widths = k_widths;
-    p.cs = cos_sin; p.cs_s0 = cs_s0; p.cs_dt = cs_dtype;
+    p.cs = cos_sin; p.cs_s0 = cs_s0;
     p.ko = (uint8_t*)key;
     p.vo = (uint16_t*)v_out; p.v_rank = v_rank;
     p.hplanes = (num_kv_heads + LIFT_WAVES - 1) / LIFT_WAVES;

@@ -19,7 +19,7 @@ import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libstarkv_hip.so")
 OPS_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libstarkv_torch.so")
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 F32, F16, BF16 = 0, 1, 2
 CACHE_Q3_2 = 16  # cache kind of the 3.2-bit QuantRow cache
@@ -101,12 +101,13 @@ def lib():
             raise RuntimeError(f"STAR-KV HIP library not built: {LIB_PATH} is missing "
                                "(run `python star-kv-serve_amd/build.py`)")
         L = ctypes.CDLL(LIB_PATH)
+        # Before the entry points: an older library may lack some.
+        if L.starkv_abi_version() != ABI_VERSION:
+            raise RuntimeError(f"{LIB_PATH}: ABI {L.starkv_abi_version()} != {ABI_VERSION}; rebuild it")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
-        if L.starkv_abi_version() != ABI_VERSION:
-            raise RuntimeError(f"{LIB_PATH}: ABI {L.starkv_abi_version()} != {ABI_VERSION}; rebuild it")
         _LIB = L
     return _LIB
 
