@@ -563,9 +563,14 @@ def test_k_up_and_v_up_dtypes_independent(cuda):
 def test_two_pass_lift_on_matrix_instructions(cuda, n, v_rank, quant):
     """More than four requests' lift of bf16 v_up_by_q: request counts around the tile of 16, rank
     columns that are no multiple of a step of 32 or of a batch, one request without tokens (NaN,
-    as the softmax over an empty row) beside the others. fp32 output against the vector form's
-    (fp16 v_up_by_q of the same values, which bf16 holds exactly): the same products, sums of
-    v_rank terms in another order."""
+    as the softmax over an empty row) beside the others. fp32 output against the float64 product of
+    the merged rows o, which a weight of unit vectors reads out (the vector form's fp16 weights: 1 o + 0).
+
+    A result is the sum of v_rank exact products; a wave's chain has up to 3 x 6 matrix products and
+    the waves' sums 8 more, each rounding by at most 2^-24 of a partial sum whose rms, for products of
+    independent signs, is at most s = sqrt(sum o^2 v^2): rms error sqrt(26) 2^-24 s, 8 with the sums
+    inside a product. Without the third part of o it is about 2^-17 / sqrt(3) s, and more without the
+    second or without the columns past the last whole step."""
     lens = [0] + [17 + 29 * i for i in range(n - 1)]
     kw = dict(num_heads=8, seed=n, v_rank=v_rank)
     wl = (W.make_quant if quant else W.make_lowrank)(lens, **kw)
@@ -573,20 +578,36 @@ def test_two_pass_lift_on_matrix_instructions(cuda, n, v_rank, quant):
     args = list(g.decode_args())
     at = [i for i, a in enumerate(args) if torch.is_tensor(a) and a.data_ptr() == g.v_up_by_q.data_ptr()][0]
     fn = paged_quant_decode if quant else paged_starkv_decode
-    v16 = g.v_up_by_q.to(torch.bfloat16).to(torch.float16)  # values both dtypes hold
-    outs = []
-    for dt in (torch.bfloat16, torch.float16):
-        args[at] = v16.to(dt)
+
+    def decode(v_up):
+        args[at] = v_up
         out = torch.empty(n, 8, 128, dtype=torch.float32, device=cuda)
         fn(*args, out=out)
-        outs.append(out.double())
-    assert torch.equal(v16.to(torch.bfloat16).double(), v16.double())
-    assert outs[0][0].isnan().all() and outs[1][0].isnan().all()
-    a, b = outs[0][1:], outs[1][1:]
-    assert torch.isfinite(a).all()
-    # Averages of normal codes: |o| <= 8. Two fp32 sums of v_rank products each.
-    bound = 2 * v_rank * 2.0 ** -24 * 8 * v16.double().abs().sum(1).max()
-    assert ((a - b).abs() <= bound).all()
+        assert out[0].isnan().all()
+        return out[1:]
+
+    unit = torch.zeros(8, 2 * v_rank + 127, 128, dtype=torch.float16, device=cuda)
+    unit[:, torch.arange(128) + v_rank - 1, torch.arange(128)] = 1  # rows r .. r + 127 from row v_rank - 1 - r on
+    o = torch.cat([decode(unit[:, v_rank - 1 - r:2 * v_rank - 1 - r].contiguous())[..., :min(128, v_rank - r)]
+                   for r in range(0, v_rank, 128)], dim=-1).double().transpose(0, 1)  # [8, n - 1, v_rank]
+    assert torch.isfinite(o).all()
+    v_up = g.v_up_by_q.to(torch.bfloat16)
+    v = v_up.double()
+    rms = lambda t: float(t.square().mean().sqrt())  # noqa: E731
+    want, bound = torch.bmm(o, v), 8 * 2.0 ** -24 * rms(torch.bmm(o.square(), v.square()).sqrt())
+    error = rms(decode(v_up).double().transpose(0, 1) - want)
+    assert error <= bound, (error, bound)
+    # What the bound has to catch: o cut to two and one of its bf16 parts, the last columns left out.
+    o32 = o.float().contiguous()
+    for part in (2, 1):
+        left, kept = o32.clone(), torch.zeros_like(o32)
+        for _ in range(part):
+            cut = (left.view(torch.int32) & -65536).view(torch.float32)
+            kept, left = kept + cut, left - cut
+        assert rms(torch.bmm(kept.double(), v) - want) > bound
+    whole = v_rank // 32 * 32
+    if whole < v_rank:
+        assert rms(torch.bmm(o[..., :whole].contiguous(), v[:, :whole].contiguous()) - want) > bound
 
 
 @pytest.mark.parametrize("n", [5, 17])

@@ -51,3 +51,31 @@ def test_lift_vs_float64(cuda, name):
     assert torch.equal(v16, v_codes.to(torch.float16))
     if dt == torch.float16:
         assert v16.data_ptr() == v_codes.data_ptr()
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_lift_bit_for_bit(cuda, name):
+    """The keys' bits: per value one fp32 chain of fused multiply-adds over the ranks, by eights in the order
+    0 2 4 6 1 3 5 7, the rotation's products and sums rounded one by one, one rounding to fp16. (A fused
+    multiply-add is formed here in float64, which holds the product, and rounded once.)"""
+    lens, widths, rv, dt, cdt = CASES[name]
+    g = torch.Generator().manual_seed(100 + len(name))
+    T, W, H = sum(lens), sum(widths), len(widths)
+    offs = [sum(widths[:h]) for h in range(H)]
+    codes = torch.randn(T, W + rv, generator=g).to(dt)
+    u = torch.randn(W, 128, generator=g) * 0.2
+    ang = torch.arange(max(lens) + 3, dtype=torch.float64)[:, None] * torch.logspace(0, -4, 64, dtype=torch.float64)
+    cs = torch.cat([ang.cos(), ang.sin()], 1).to(cdt)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda)  # noqa: E731
+    dev = codes.to(cuda)
+    key = prefill_lift(dev[:, :W], dev[:, W:], prompt_tables(lens, cuda)[0], u.to(cuda), i32(offs), i32(widths), cs.to(cuda))[0]
+    c, s = cs[torch.cat([torch.arange(L) for L in lens])].float().chunk(2, 1)
+    for h in range(H):
+        x = torch.zeros(T, 128)
+        for r0 in range(0, widths[h], 8):
+            for r in (r0 + i for i in (0, 2, 4, 6, 1, 3, 5, 7)):
+                if r < widths[h]:
+                    x = (x.double() + codes[:, offs[h] + r, None].double() * u[offs[h] + r].double()).float()
+        x1, x2 = x.chunk(2, 1)
+        want = torch.cat([x1 * c - x2 * s, x2 * c + x1 * s], 1).to(torch.float16)
+        assert torch.equal(key[:, h].cpu().view(torch.int16), want.view(torch.int16)), f"{name}: head {h}"
