@@ -184,7 +184,8 @@ class StarKVLlamaForCausalLM:
             kc, vc = self.kv_caches[li]
             ka, va = k, v  # the prefill attention's operands
             slots = md.slot_mapping[:T]
-            if model_ops.rope_write_fits(self.rotary.cos_sin_cache, positions, q, k, v, kc, vc, slots):
+            own = getattr(self.rotary.apply, "__func__", None) is Rotary.apply  # not a rotation of the caller's
+            if own and model_ops.rope_write_fits(self.rotary.cos_sin_cache, positions, q, k, v, kc, vc, slots):
                 q, k, ka, va = model_ops.rope_write(positions, q, k, v, self.rotary.cos_sin_cache, kc, vc, slots,
                                                     capture is not None, bool(md.num_prefills))
             else:

@@ -433,3 +433,23 @@ def test_stock_decode_splits_by_own_length(cuda, H, span, lens):
         truth[i] = torch.einsum("hl,lhd->hd", p, V)
     assert_close(out[live], truth.cpu().numpy(), f"own splits H={H} n={n}")
     assert all(bool(out[b].isnan().all()) for b in range(n) if not lens[b])
+
+
+def test_a_rotation_of_the_callers_is_used(cuda):
+    """A model whose rotary is replaced rotates with that one's apply in every layer, also where the kernel could."""
+    class Half(M.Rotary):
+        def apply(self, positions, x):
+            return super().apply(positions, x) * 0.5
+
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, seed=2)
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    pos, tokens = torch.tensor([3, 5], device=cuda), torch.tensor([1, 2], device=cuda)
+    model.rotary = Half(65, torch.bfloat16, cuda, 10000.0)
+    model.allocate_kv_cache(9)
+    cap = []
+    model.decode_step(tokens, pos, M.decode_metadata(bt, pos, 16, 6), capture=cap)
+    kc = model.kv_caches[0][0]
+    assert torch.equal(kc[bt[:, 0].long(), pos], cap[0]["k"])
+    h = cap[0]["h"].float() @ model.layers[0].qkv_proj.float().T
+    k = M.Rotary.apply(model.rotary, pos, h[:, 512:1024].view(2, 4, 128)) * 0.5
+    torch.testing.assert_close(cap[0]["k"].float(), k, rtol=0, atol=3 * 2.0 ** -8 * float(k.abs().max()))  # three roundings
