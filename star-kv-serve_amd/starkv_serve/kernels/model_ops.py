@@ -105,6 +105,12 @@ def decode_slots(block_table: torch.Tensor, positions: torch.Tensor, block_size:
     return slots, lens
 
 
+def greedy_fits(logits: torch.Tensor, tokens: torch.Tensor) -> bool:
+    """Whether ``greedy_step`` takes these logits: rows that 16-byte loads can take."""
+    return (tokens.dtype == torch.int64 and logits.dtype in _FLOATS and logits.stride(1) == 1
+            and logits.stride(0) % 8 == 0 and logits.data_ptr() % 16 == 0)
+
+
 def greedy_step(logits: torch.Tensor, tokens: torch.Tensor, positions: torch.Tensor) -> None:
     """tokens [n] = logits.argmax(-1) (the first of equals), positions [n] += 1, in place."""
     _hip.ops().greedy_step(logits, tokens, positions)

@@ -340,7 +340,7 @@ class DecodeGraph:
         m = self.model
         md = decode_metadata(self.block_table, self.positions, m.block_size, m.max_model_len)
         self.logits = m.decode_step(self.tokens, self.positions, md, in_graph=True)
-        if self.tokens.dtype == torch.int64 and m.shape.vocab_size % 8 == 0:
+        if model_ops.greedy_fits(self.logits, self.tokens):
             model_ops.greedy_step(self.logits, self.tokens, self.positions)
         else:
             self.tokens.copy_(self.logits.argmax(-1))

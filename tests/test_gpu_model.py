@@ -453,3 +453,18 @@ def test_a_rotation_of_the_callers_is_used(cuda):
     h = cap[0]["h"].float() @ model.layers[0].qkv_proj.float().T
     k = M.Rotary.apply(model.rotary, pos, h[:, 512:1024].view(2, 4, 128)) * 0.5
     torch.testing.assert_close(cap[0]["k"].float(), k, rtol=0, atol=3 * 2.0 ** -8 * float(k.abs().max()))  # three roundings
+
+
+def test_decode_graph_takes_a_head_of_any_width(cuda):
+    """A head with more rows than the vocabulary, an odd number of them: the graph's tokens are the logits'
+    argmax, replay by replay."""
+    model = M.StarKVLlamaForCausalLM(SHAPE, None, max_model_len=64, device=cuda, seed=2)
+    model.allocate_kv_cache(9)
+    model.lm_head, model.embed = (torch.cat([t, t[:1] * 2]) for t in (model.lm_head, model.embed))
+    bt = torch.arange(1, 9, device=cuda, dtype=torch.int32).view(2, 4)
+    graph = M.DecodeGraph(model, bt, torch.tensor([1, 2], device=cuda), torch.tensor([3, 5], device=cuda))
+    for step in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert graph.logits.shape == (2, 1001) and torch.equal(graph.tokens, graph.logits.argmax(-1))
+        assert graph.positions.tolist() == [4 + step, 6 + step]
