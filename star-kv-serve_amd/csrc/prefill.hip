@@ -32,7 +32,7 @@
 // the matrix unit with its power: 64 % busy, 983 TFLOP/s at one 16,384-token prompt of 32 heads
 // where a large bf16 product of the library reaches 1242. Scores, softmax and P @ V one after the
 // other, a swizzle whose V reads met in one bank quarter, and heads spread over the XCDs took
-// 3214 us there against 2237 now; 4096 tokens 291 against 158, 2048 tokens 82 against 53.
+// 3214 us there against 2237 now, on one box; 4096 tokens 291 against 158, 2048 tokens 82 against 53.
 // At the end the two halves of each query's sum are added and O / l is written.
 #include <algorithm>
 #include <array>
